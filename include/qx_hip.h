@@ -356,9 +356,10 @@ QXH_API int32_t qxh_encode_attention_for_layer_no_alloc(qxh_graph* graph, qxh_kv
  * layer's V rows [0, start_position + tokens) into an f16 V^T scratch inside
  * `workspace` (Granite-shape f16 caches are read as they are).  For bf16
  * caches, rows that reach a V value outside the f16 range are recomputed by
- * an exact bf16 pass.  Granite-shape fp32 and mixed caches run an fp32
- * matrix-core kernel (fp32 products and accumulation); Qwen-shape fp32
- * caches run causal decode rows.  `workspace` must hold
+ * an exact bf16 pass.  Granite-shape fp32 and mixed caches run a
+ * kernel that splits each fp32 operand into 16-bit pieces holding all 24
+ * bits (fp32 accuracy and accumulation); Qwen-shape fp32 caches run causal
+ * decode rows.  `workspace` must hold
  * qxh_prefill_workspace_bytes, which covers every start_position: the V^T
  * scratch where it is used (kv_heads x capacity rounded up to 64 x head_dim
  * x 2 bytes plus per-tile flags) and the split partials, for decode rows the

@@ -39,6 +39,22 @@ template <> struct MfmaT<BF16> {
 
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 
+// Four consecutive elements in one store (16 or 8 bytes), rounded as
+// store_any rounds them; the address needs the element's alignment only.
+__device__ __forceinline__ void store4_any(void* p, size_t i, const f32x4& v, int dt) {
+    typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+    typedef uint16_t u16x4_u __attribute__((ext_vector_type(4), aligned(2)));
+    if (dt == F32) {
+        *reinterpret_cast<f32x4_u*>(reinterpret_cast<float*>(p) + i) = v;
+        return;
+    }
+    u16x4_u w;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        w[j] = dt == F16 ? __builtin_bit_cast(uint16_t, from_f32<F16>(v[j])) : from_f32<BF16>(v[j]).bits;
+    *reinterpret_cast<u16x4_u*>(reinterpret_cast<uint16_t*>(p) + i) = w;
+}
+
 // Reductions across the four 16-lane groups (which hold the same query column
 // at different positions).  v_permlane{16,32}_swap exchange lane halves on
 // the VALU; with both operands equal, op(result[0], result[1]) is

@@ -50,8 +50,12 @@ constexpr uint32_t kExactPassWgs = 256;
 //   4000 + 12 15.4 / 13.7, 0 + 9 7.7 / 5.9;
 // - Granite bf16 (c = 0, 90000): 3000 + 32 17.1 / 19.1, 2000 + 48 21.7 /
 //   18.2, 8000 + 9 18.5 / 24.5, 8000 + 16 25.3 / 24.2;
-// - the Granite fp32 matrix-core kernel (fp32 and mixed caches; c = 0,
-//   70000): Fp32KFp16V 4000 + 16 19.6 / 22.1, 1500 + 48 23.9 / 21.5;
+// - the Granite split-product kernel (fp32 and mixed caches; c = 0, 22000):
+//   Fp32KFp16V 1000 + 16 10.4 / 11.0, 500 + 32 12.1 / 12.9, 2000 + 9 13.6 /
+//   12.3, 1000 + 24 14.1 / 11.4, 500 + 48 14.4 / 13.2; fp32 K/V 500 + 48
+//   15.0 / 16.6, 1000 + 24 14.9 / 13.4; Fp16KFp32V 2000 + 9 13.2 / 13.7,
+//   1000 + 24 13.4 / 12.7 (70000 while it ran on the fp32 matrix cores:
+//   4000 + 16 22.2 / 15.6 went to the rows);
 // - the other Granite plans (tiered values): c = 0, 40000;
 // - Qwen with tiered values (c = 0, 150000), whose decode rows keep splits
 //   toward 2048 workgroups.
@@ -64,7 +68,7 @@ static bool rows_on_decode(const ShapeDims& s, int key_dtype, int value_dtype, u
     const uint64_t length = (uint64_t)start + tokens;
     if (s.group >= 8)
         return value_dtype == I8T ? tokens * length <= 150000u : (tokens - 6) * length <= 126000u;
-    if (prefill_f32_supported(s, key_dtype, value_dtype)) return tokens * length <= 70000u;
+    if (prefill_f32_supported(s, key_dtype, value_dtype)) return tokens * length <= 22000u;
     if (key_dtype == F16 && value_dtype == F16) return start >= 64 && tokens * length <= 70000u;
     if (key_dtype == BF16 && value_dtype == BF16) return tokens * length <= 90000u;
     return tokens * length <= 40000u;
@@ -76,7 +80,7 @@ static bool prefill_on_decode(const ShapeDims& s, int key_dtype, int value_dtype
 }
 
 // fp32 and mixed K/V caches at the Granite shape beyond a few rows take the
-// fp32 matrix-core kernel (prefill_f32.hip); Qwen-shape fp32 caches and
+// split-product kernel (prefill_f32.hip); Qwen-shape fp32 caches and
 // tiered values stay on causal decode rows.
 static bool prefill_on_f32(const ShapeDims& s, int key_dtype, int value_dtype, uint32_t start, uint32_t tokens) {
     return prefill_f32_supported(s, key_dtype, value_dtype) && !rows_on_decode(s, key_dtype, value_dtype, start, tokens);

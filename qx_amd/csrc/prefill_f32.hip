@@ -1,35 +1,54 @@
 // Causal prefill on fp32 and mixed K/V caches at the Granite shape (16 q /
 // 8 kv heads, d 64): the reference's KV plans Fp32KFp16V (its default) and
-// Fp16KFp32V, fp32 K/V, and their bf16 twins.  fp32 accuracy rules out the
-// 16-bit matrix products of the pipelined kernel, so both products run on
-// the fp32 matrix cores (v_mfma_f32_16x16x4_f32, fp32 in and out) in the
-// transposed FlashAttention-2 form:
+// Fp16KFp32V, fp32 K/V, their bf16 twins, and fp32 keys with tiered values.
+// fp32 accuracy rules out rounding an operand to 16 bits, and the fp32 matrix
+// cores run at a sixteenth of the 16-bit rate, so every fp32 operand is split
+// into 16-bit pieces that hold all of its 24 significand bits, and each
+// product is the sum of the piece products that matter:
 //
-//   S^T[pos][q]  = K[pos][:] . Q^T[:][q]       A = K tile (LDS), B = Q^T (registers)
-//   O^T[d][q]   += V^T[d][pos] . P^T[pos][q]    A = V tile (LDS), B = P^T (registers)
+//   x = x0 + x1 + x2      bf16: x0 the top 8 bits, x1 and x2 the remainders
+//                         rounded to nearest; f16 values are two pieces and
+//                         bf16 values one, exactly
+//   x . y = sum of xi . yj with i + j <= 2 (what is left out is below 2^-24
+//                         of the product), accumulated in fp32, the small
+//                         products first
 //
-// 16x16x4 f32 operand layout (lane l, g = l / 16, i = l % 16): A[m][k] from
-// lane m + 16k, B[k][n] from lane n + 16k, D[m][n] in lane n + 16(m / 4),
-// element m % 4.  A contraction may number its k slots in any order as long
-// as A and B agree, so:
-//   * S^T, MFMA step s (0..15) contracts dims {16g + s}: lane (g, i) supplies
-//     K[pos i][16g + s] and Q[column i][16g + s], i.e. 16 consecutive dims of
-//     one row each (four 16-byte LDS reads of K per 16-position block);
-//   * P.V, MFMA (pb, j) contracts positions {16 pb + 4g + j}: exactly the
-//     probabilities the S^T block pb leaves in lane (g, i) as element j, so
-//     P^T needs no exchange; lane (g, i) supplies V[16 pb + 4g + j][4i + db]
-//     for output block db (0..3), one 16-byte LDS read serving all four, and
-//     O^T block db row m is dim 4m + db.
+// Probabilities over f16 values (exact as they are) are two f16 pieces, held
+// to 2^-23; their exponent is offset by 2^12 so that the second piece stays
+// clear of f16's subnormals.  Against 64 bits the result is as close as the
+// fp32 matrix cores' was or closer (1900 tokens: 2.6e-7 of the result against
+// 3.3e-7 on Fp32KFp16V; 3000 tokens of fp32 K/V: 3.5e-7 against 4.6e-7).
+//
+// Bound: at 1900 tokens of Fp32KFp16V 128 MFMAs a tile and wave (2048 cycles
+// of matrix core; 8192 on the fp32 cores) run in about 45 us, against 88 on
+// the fp32 cores; the matrix core is busy a quarter of that, the rest is the
+// softmax and the split of the tile on the VALU, waits, and the start of each
+// workgroup (query pieces, first tile).
+//
+// Transposed FlashAttention-2 on 16x16x32 MFMAs (operand layout: mfma.h):
+//
+//   S^T[pos][q]  = K[pos][:] . Q^T[:][q]       A = K pieces (LDS), B = Q^T pieces (registers)
+//   O^T[d][q]   += V^T[d][pos] . P^T[pos][q]    A = V pieces (LDS, transposed reads), B = P^T pieces
+//
+// The S^T blocks leave in lane (g, i) exactly the positions that the
+// transposed V reads (vt_operand_rows32) give it, so P^T needs no exchange.
 //
 // A workgroup of 4 waves owns a query block of 64 tokens x the 2 heads of a
 // kv head (128 columns; wave w: tokens 16w .. 16w + 15, both heads), the
 // column layout of the pipelined Granite kernel, so its split-KV partials go
 // through the same prefill_combine_kernel.  K and V tiles of 64 positions are
-// read with 16-byte loads (whole tile per load instruction), widened to fp32
-// and written to a double-buffered, padded LDS ring; the next tile's loads
-// are in flight while the current one is computed.  Scores are scaled by
-// softmax scale x log2(e) in fp32 after the dot product and exponentiated
-// with v_exp_f32; the online softmax keeps per-column (m, l) in every lane.
+// read with 16-byte loads, split once per workgroup and written to LDS as one
+// 8 KB plane per piece, 16-byte chunks XOR-swizzled by row & 7 (conflict-free
+// for both kinds of operand read); the next tile's loads are in flight while
+// the current one is computed.  Scores are scaled by softmax scale x log2(e)
+// in fp32 after the dot product and exponentiated with v_exp_f32; the online
+// softmax keeps per-column (m, l) in every lane.
+//
+// A piece of an infinity, or a product that overflows where the whole one
+// does not, would turn into a NaN, so a workgroup that meets a magnitude of
+// 2^60 or more (a non-finite f16 value, say) takes that tile's two products
+// on the fp32 matrix cores, straight from the cache.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -42,47 +61,120 @@ namespace qxh {
 namespace {
 
 constexpr int kD = 64;
-constexpr int kRowF = kD + 4;                  // padded fp32 row of a staged tile (floats)
-constexpr int kTileF = kPrefillTile * kRowF;   // floats per staged tile
 constexpr float kNegBigF = -1.0e30f;
-constexpr int kTierBlockF32 = 32;  // elements per INT8 scale block of a tiered value cache
+constexpr int kTierBlockF32 = 32;           // elements per INT8 scale block of a tiered value cache
+constexpr int kPlaneBytes = kPrefillTile * kD * 2;
+constexpr float kSplitLimit = 0x1p60f;      // magnitudes the split products take
 
 __device__ __forceinline__ f32x4 mma4(float a, float b, const f32x4& c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// A 64 x 64 tile of one dtype moved as 16-byte chunks: chunk k of thread t
-// holds elements EPC (t + 256 k) .. + EPC - 1 of the tile in row-major order
-// (EPC = 4 for fp32, 8 for 16-bit), so each load instruction of the
-// workgroup reads the tile's bytes contiguously.
-template <int DT> struct TileIo {
-    static constexpr int EB = DT == F32 ? 4 : 2;
-    static constexpr int EPC = 16 / EB;
-    static constexpr int CH = kPrefillTile * kD / EPC / 256;  // chunks per thread
-    // rows at or past kv_len read the last row instead (their positions are masked)
-    __device__ __forceinline__ static void load(u32x4 (&raw)[CH], const char* base, uint32_t tile, uint32_t kv_len,
-                                                int tid) {
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+// bf16 pieces of the pair (a, b), packed (a in the low half).  x0 is cut off,
+// not rounded: the pieces of a finite value are finite.
+__device__ __forceinline__ uint32_t top_bf16(float& a, float& b) {
+    const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
+    const uint32_t w = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
+    a -= __uint_as_float(ua & 0xffff0000u);
+    b -= __uint_as_float(ub & 0xffff0000u);
+    return w;
+}
+__device__ __forceinline__ uint32_t round_bf16(float& a, float& b) {
+    const uint32_t w = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)a, (__bf16)b});
+    a -= __uint_as_float(w << 16);
+    b -= __uint_as_float(w & 0xffff0000u);
+    return w;
+}
+
+// 8 values as NP packed bf16 pieces (the values are used up).
+template <int NP> __device__ __forceinline__ void split8(float (&f)[8], u32x4 (&p)[NP]) {
 #pragma unroll
-        for (int k = 0; k < CH; ++k) {
-            const int e = EPC * (tid + 256 * k);
-            const uint32_t row = min(tile * kPrefillTile + (uint32_t)(e / kD), kv_len - 1);
-            raw[k] = load16<false>(base + ((size_t)row * kD + e % kD) * EB);
+    for (int i = 0; i < 4; ++i) {
+        p[0][i] = top_bf16(f[2 * i], f[2 * i + 1]);
+        if constexpr (NP > 1) p[1][i] = round_bf16(f[2 * i], f[2 * i + 1]);
+        if constexpr (NP > 2) p[2][i] = round_bf16(f[2 * i], f[2 * i + 1]);
+    }
+}
+
+// f16 pieces of the pair (a, b): the pair rounded to nearest, and what that
+// left of it (exact before its own rounding; one v_fma_mix per value).
+__device__ __forceinline__ uint32_t round_f16(float a, float b, uint32_t& rest) {
+    const uint32_t w = __builtin_bit_cast(uint32_t, f16x2{(_Float16)a, (_Float16)b});
+    uint32_t r;
+    asm("v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]\n\t"
+        "v_fma_mixhi_f16 %0, %1, -1.0, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+        : "=&v"(r)
+        : "v"(w), "v"(a), "v"(b));
+    rest = r;
+    return w;
+}
+
+__device__ __forceinline__ float max_abs8(const float (&f)[8], float m) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m = fmaxf(m, __builtin_fabsf(f[i]));
+    return m;
+}
+
+// Byte offset of 16-byte chunk `col` of tile row `row` in a plane.
+__device__ __forceinline__ int plane_chunk(int row, int col) { return row * (kD * 2) + ((col ^ (row & 7)) << 4); }
+
+// A 64 x 64 tile of one dtype: thread t moves chunks of 8 elements, chunk k at
+// row t / 8 + 32 k, elements 8 (t % 8) .. + 7.  PIECES planes; as values an
+// f16 tile stays f16 (VALUES), as keys it is two bf16 pieces.
+template <int DT, bool VALUES> struct SplitIo {
+    static constexpr int EB = DT == F32 ? 4 : 2;
+    static constexpr int PIECES = DT == F32 ? 3 : DT == F16 && !VALUES ? 2 : 1;
+    static constexpr int WORDS = DT == F32 ? 2 : 1;  // 16-byte loads a chunk
+    struct Raw {
+        u32x4 w[2][WORDS];
+    };
+    // rows at or past kv_len read the last row instead (their positions are masked)
+    __device__ __forceinline__ static void load(Raw& raw, const char* base, uint32_t tile, uint32_t kv_len, int tid) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const uint32_t row = min(tile * kPrefillTile + (uint32_t)(tid >> 3) + 32 * k, kv_len - 1);
+            const char* p = base + ((size_t)row * kD + 8 * (tid & 7)) * EB;
+#pragma unroll
+            for (int i = 0; i < WORDS; ++i) raw.w[k][i] = load16<false>(p + 16 * i);
         }
     }
-    __device__ __forceinline__ static void store(const u32x4 (&raw)[CH], float* lds, int tid) {
+    // returns whether a magnitude reaches the split's limit
+    __device__ __forceinline__ static bool store(const Raw& raw, char* lds, int tid) {
+        float m = 0.0f;
 #pragma unroll
-        for (int k = 0; k < CH; ++k) {
-            const int e = EPC * (tid + 256 * k);
-            float* dst = lds + (e / kD) * kRowF + e % kD;
+        for (int k = 0; k < 2; ++k) {
+            char* dst = lds + plane_chunk((tid >> 3) + 32 * k, tid & 7);
+            float f[8];
             if constexpr (DT == F32) {
-                *reinterpret_cast<u32x4*>(dst) = raw[k];
+                float lo[4], hi[4];
+                Unpack<F32>::run(raw.w[k][0], lo);
+                Unpack<F32>::run(raw.w[k][WORDS - 1], hi);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    f[i] = lo[i];
+                    f[4 + i] = hi[i];
+                }
             } else {
-                float f[8];
-                Unpack<DT>::run(raw[k], f);
-                *reinterpret_cast<f32x4*>(dst) = f32x4{f[0], f[1], f[2], f[3]};
-                *reinterpret_cast<f32x4*>(dst + 4) = f32x4{f[4], f[5], f[6], f[7]};
+                Unpack<DT>::run(raw.w[k][0], f);
+            }
+            m = max_abs8(f, m);
+            if constexpr (PIECES == 1) {
+                *reinterpret_cast<u32x4*>(dst) = raw.w[k][0];
+            } else {
+                u32x4 p[PIECES];
+                split8<PIECES>(f, p);
+#pragma unroll
+                for (int i = 0; i < PIECES; ++i) *reinterpret_cast<u32x4*>(dst + i * kPlaneBytes) = p[i];
             }
         }
+        return m >= (DT == F16 ? 65536.0f : kSplitLimit);
+    }
+    __device__ __forceinline__ static float at(const PrefillPipeArgs&, const char* base, uint32_t, uint32_t row,
+                                               int dim) {
+        return load_f32<DT>(base, (size_t)row * kD + dim);
     }
 };
 
@@ -90,78 +182,70 @@ template <int DT> struct TileIo {
 // .. + 15 of row t / 4 (half of one 32-element block).  A row below the
 // boundary is 16 INT8 codes times the block's f16 scale (exact in fp32), a
 // row at or above it 16 f16 values from its window slot.
-struct TieredTileIo {
+struct TieredSplitIo {
     static constexpr int EB = 1;  // bytes per element of `values` (the INT8 codes)
-    static constexpr int CH = 2;
+    static constexpr int PIECES = 3;
+    struct Raw {
+        u32x4 w[2];
+    };
     __device__ __forceinline__ static uint32_t row_of(uint32_t tile, uint32_t kv_len, int tid) {
         return min(tile * kPrefillTile + (uint32_t)(tid >> 2), kv_len - 1);
     }
-    __device__ __forceinline__ static void load(u32x4 (&raw)[CH], const PrefillPipeArgs& a, uint32_t kvh,
-                                                uint32_t tile, uint32_t kv_len, int tid) {
+    __device__ __forceinline__ static void load(Raw& raw, const PrefillPipeArgs& a, uint32_t kvh, uint32_t tile,
+                                                uint32_t kv_len, int tid) {
         const uint32_t row = row_of(tile, kv_len, tid);
         const int col = 16 * (tid & 3);
         if (row < a.tier) {
             const size_t e = (size_t)kvh * a.head_stride + (size_t)row * kD + col;
-            raw[0] = load16<false>(reinterpret_cast<const int8_t*>(a.values) + e);
-            raw[1] = u32x4{(uint32_t)a.value_scales[e / kTierBlockF32], 0u, 0u, 0u};
+            raw.w[0] = load16<false>(reinterpret_cast<const int8_t*>(a.values) + e);
+            raw.w[1] = u32x4{(uint32_t)a.value_scales[e / kTierBlockF32], 0u, 0u, 0u};
         } else {
             const uint16_t* w =
                 a.value_ring + (size_t)kvh * a.ring_head_stride + (size_t)(row & a.window_mask) * kD + col;
-            raw[0] = load16<false>(w);
-            raw[1] = load16<false>(w + 8);
+            raw.w[0] = load16<false>(w);
+            raw.w[1] = load16<false>(w + 8);
         }
     }
-    __device__ __forceinline__ static void store(const u32x4 (&raw)[CH], float* lds, const PrefillPipeArgs& a,
-                                                 uint32_t tile, uint32_t kv_len, int tid) {
-        float f[16];
+    __device__ __forceinline__ static bool store(const Raw& raw, char* lds, const PrefillPipeArgs& a, uint32_t tile,
+                                                 uint32_t kv_len, int tid) {
+        float f[2][8];
         if (row_of(tile, kv_len, tid) < a.tier) {
-            const float sc = (float)__builtin_bit_cast(half_t, (uint16_t)raw[1][0]);
+            const float sc = (float)__builtin_bit_cast(half_t, (uint16_t)raw.w[1][0]);
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                const int32_t code = (int32_t)(raw[0][i >> 2] << (24 - 8 * (i & 3))) >> 24;
-                f[i] = (float)code * sc;
+                const int32_t code = (int32_t)(raw.w[0][i >> 2] << (24 - 8 * (i & 3))) >> 24;
+                f[i >> 3][i & 7] = (float)code * sc;
             }
         } else {
-            Unpack<F16>::run(raw[0], f);
-            float g[8];
-            Unpack<F16>::run(raw[1], g);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) f[8 + i] = g[i];
+            Unpack<F16>::run(raw.w[0], f[0]);
+            Unpack<F16>::run(raw.w[1], f[1]);
         }
-        float* dst = lds + (tid >> 2) * kRowF + 16 * (tid & 3);
+        float m = 0.0f;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            *reinterpret_cast<f32x4*>(dst + 4 * r) = f32x4{f[4 * r], f[4 * r + 1], f[4 * r + 2], f[4 * r + 3]};
+        for (int k = 0; k < 2; ++k) {
+            m = max_abs8(f[k], m);
+            u32x4 p[3];
+            split8<3>(f[k], p);
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                *reinterpret_cast<u32x4*>(lds + i * kPlaneBytes + plane_chunk(tid >> 2, 2 * (tid & 3) + k)) = p[i];
+        }
+        return m >= kSplitLimit;
+    }
+    __device__ __forceinline__ static float at(const PrefillPipeArgs& a, const char*, uint32_t kvh, uint32_t row,
+                                               int dim) {
+        if (row < a.tier) {
+            const size_t e = (size_t)kvh * a.head_stride + (size_t)row * kD + dim;
+            return (float)reinterpret_cast<const int8_t*>(a.values)[e] *
+                   (float)__builtin_bit_cast(half_t, a.value_scales[e / kTierBlockF32]);
+        }
+        return (float)__builtin_bit_cast(
+            half_t, a.value_ring[(size_t)kvh * a.ring_head_stride + (size_t)(row & a.window_mask) * kD + dim]);
     }
 };
 
-// 16 consecutive elements of a query row in its dtype, widened.
-__device__ __forceinline__ void load_q16(const void* base, size_t idx, int dt, float (&q)[16]) {
-    if (dt == F32) {
-        const float* p = reinterpret_cast<const float*>(base) + idx;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const u32x4 v = load16<false>(p + 4 * r);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) q[4 * r + e] = __uint_as_float(v[e]);
-        }
-        return;
-    }
-    const uint16_t* p = reinterpret_cast<const uint16_t*>(base) + idx;
-    const u32x4 v0 = load16<false>(p), v1 = load16<false>(p + 8);
-    float lo[8], hi[8];
-    if (dt == F16) {
-        Unpack<F16>::run(v0, lo);
-        Unpack<F16>::run(v1, hi);
-    } else {
-        Unpack<BF16>::run(v0, lo);
-        Unpack<BF16>::run(v1, hi);
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        q[e] = lo[e];
-        q[8 + e] = hi[e];
-    }
+__device__ __forceinline__ f32x4 mma_bf(const u32x4& a, const u32x4& b, const f32x4& c) {
+    return MfmaT<BF16>::mma(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c);
 }
 
 }  // namespace
@@ -169,9 +253,16 @@ __device__ __forceinline__ void load_q16(const void* base, size_t idx, int dt, f
 // grid (qblocks x kv_heads, chunks of the longest block), block 256.
 template <int KDT, int VDT>
 __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) {
-    using KIo = TileIo<KDT>;
-    using VIo = std::conditional_t<VDT == I8T, TieredTileIo, TileIo<VDT == I8T ? F16 : VDT>>;
-    __shared__ __attribute__((aligned(16))) float lds[2][2][kTileF];  // [stage][K, V]
+    using KIo = SplitIo<KDT, false>;
+    using VIo = std::conditional_t<VDT == I8T, TieredSplitIo, SplitIo<VDT == I8T ? F16 : VDT, true>>;
+    constexpr int NK = KIo::PIECES, NV = VIo::PIECES;
+    constexpr bool kHalfV = VDT == F16;
+    constexpr float kShift = kHalfV ? 12.0f : 0.0f;  // exponent offset of the probabilities
+    constexpr int kStageBytes = (NK + NV) * kPlaneBytes;
+    // two stages where two workgroups of them still share a CU's 160 KB
+    constexpr int STAGES = kStageBytes < 40 * 1024 ? 2 : 1;
+    __shared__ __attribute__((aligned(16))) char lds[STAGES][kStageBytes];
+    __shared__ __attribute__((aligned(16))) uint32_t wide[2][4];  // [tile parity][wave]: the tile exceeds the split
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -215,79 +306,148 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
     const char* kbase = reinterpret_cast<const char*>(a.keys) + (size_t)kvh * a.head_stride * KIo::EB;
     const char* vbase = reinterpret_cast<const char*>(a.values) + (size_t)kvh * a.head_stride * VIo::EB;
 
-    auto vload = [&](u32x4 (&raw)[VIo::CH], uint32_t tile) __attribute__((always_inline)) {
-        if constexpr (VDT == I8T) VIo::load(raw, a, kvh, tile, kv_len, tid);
-        else VIo::load(raw, vbase, tile, kv_len, tid);
+    typename KIo::Raw kraw;
+    typename VIo::Raw vraw;
+    auto load_tile = [&](uint32_t tile) __attribute__((always_inline)) {
+        KIo::load(kraw, kbase, tile, kv_len, tid);
+        if constexpr (VDT == I8T) VIo::load(vraw, a, kvh, tile, kv_len, tid);
+        else VIo::load(vraw, vbase, tile, kv_len, tid);
     };
-    auto vstore = [&](const u32x4 (&raw)[VIo::CH], float* dst, uint32_t tile) __attribute__((always_inline)) {
-        if constexpr (VDT == I8T) VIo::store(raw, dst, a, tile, kv_len, tid);
-        else VIo::store(raw, dst, tid);
+    bool qwide = false;
+    auto store_tile = [&](uint32_t tile, uint32_t r) __attribute__((always_inline)) {
+        char* dst = lds[r % STAGES];
+        bool w = KIo::store(kraw, dst, tid);
+        if constexpr (VDT == I8T) w |= VIo::store(vraw, dst + NK * kPlaneBytes, a, tile, kv_len, tid);
+        else w |= VIo::store(vraw, dst + NK * kPlaneBytes, tid);
+        const uint32_t any = __any(w | qwide) ? 1u : 0u;
+        if (lane == 0) wide[r & 1][wave] = any;
     };
 
-    // tile 0 of the chunk into stage 0; the query loads go out behind it
-    u32x4 kraw[KIo::CH], vraw[VIo::CH];
-    KIo::load(kraw, kbase, t0, kv_len, tid);
-    vload(vraw, t0);
-
-    // Q^T operands: lane (g, i) holds dims 16g .. 16g + 15 of column i
-    float q[2][16];
+    // The query goes out before the chunk's first tile: loads complete in
+    // order, so its pieces are formed while the tile is in flight.
+    // Q^T pieces: lane (g, i) holds dims 32h + 8g .. + 7 of column i
+    u32x4 q[2][2][3];  // [head][h][piece]
     {
-        const uint32_t qr = min(tok, T - 1);
+        const size_t qrow = ((size_t)min(tok, T - 1) * a.q_heads + (size_t)kvh * 2) * kD + 8 * lg;
+        u32x4 raw[4][2];
+        if (a.query_dtype == F32) {
+            const float* p = reinterpret_cast<const float*>(a.query) + qrow;
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt)
-            load_q16(a.query, ((size_t)qr * a.q_heads + (size_t)kvh * 2 + nt) * kD + 16 * lg, a.query_dtype, q[nt]);
+            for (int x = 0; x < 8; ++x) raw[x >> 1][x & 1] = load16<false>(p + 32 * (x >> 1) + 4 * (x & 1));
+        } else {
+            const uint16_t* p = reinterpret_cast<const uint16_t*>(a.query) + qrow;
+#pragma unroll
+            for (int x = 0; x < 4; ++x) raw[x][0] = raw[x][1] = load16<false>(p + 32 * x);
+        }
+        load_tile(t0);
+        __builtin_amdgcn_sched_barrier(0);
+        float mq = 0.0f;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            float f[8];
+            if (a.query_dtype == F32) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) f[e] = __uint_as_float(raw[x][e >> 2][e & 3]);
+            } else if (a.query_dtype == F16) {
+                Unpack<F16>::run(raw[x][0], f);
+            } else {
+                Unpack<BF16>::run(raw[x][0], f);
+            }
+            mq = max_abs8(f, mq);
+            split8<3>(f, q[x >> 1][x & 1]);
+        }
+        qwide = mq >= kSplitLimit;
     }
-    KIo::store(kraw, lds[0][0], tid);
-    vstore(vraw, lds[0][1], t0);
+    store_tile(t0, 0);
     __syncthreads();
 
-    f32x4 oacc[4][2];  // [output block db][head nt]
+    f32x4 oacc[4][2];  // [output block db][head nt]: lane (g, i) holds dims 16db + 4g + j of column i
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) oacc[db][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
     float mrun[2] = {kNegBigF, kNegBigF}, lsum[2] = {0.f, 0.f};
 
-    auto compute = [&](const float* Kl, const float* Vl, uint32_t kt) __attribute__((always_inline)) {
+    // operand addresses inside a stage: K rows 16 pb + i, chunk 4 h + g; V
+    // rows 32 h + 4 g + i / 4 (+ 16), dims 16 db + 4 (i % 4)
+    const int k_off = plane_chunk(li, lg);
+    const int v_row = 4 * lg + (li >> 2);
+
+    auto compute = [&](const char* st, uint32_t kt, bool split) __attribute__((always_inline)) {
+        int l = lane;  // the lane number as the fp32 path sees it
+        if (!split) asm volatile("" : "+v"(l));  // nothing of it is computed (and held in registers) outside it
         // S^T = K . Q^T, four 16-position blocks
         f32x4 sacc[4][2];
+        if (split) {
 #pragma unroll
-        for (int pb = 0; pb < 4; ++pb) {
-            const float* kr = Kl + (16 * pb + li) * kRowF + 16 * lg;
-            f32x4 k4[4];
+            for (int pb = 0; pb < 4; ++pb) {
+                f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+                u32x4 k[2][NK];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) k4[r] = *reinterpret_cast<const f32x4*>(kr + 4 * r);
+                for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int nt = 0; nt < 2; ++nt) {
-                f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+                    for (int i = 0; i < NK; ++i)
+                        k[h][i] = *reinterpret_cast<const u32x4*>(st + i * kPlaneBytes + pb * 16 * kD * 2 +
+                                                                  (k_off ^ (h * 64)));
 #pragma unroll
-                for (int s = 0; s < 16; ++s) acc = mma4(k4[s >> 2][s & 3], q[nt][s], acc);
-                sacc[pb][nt] = acc;
+                for (int sum = 2; sum >= 0; --sum)  // the small products first
+#pragma unroll
+                    for (int i = 0; i < NK; ++i)
+#pragma unroll
+                        for (int h = 0; h < 2; ++h)
+#pragma unroll
+                            for (int nt = 0; nt < 2; ++nt)
+                                if (i <= sum) acc[nt] = mma_bf(k[h][i], q[nt][h][sum - i], acc[nt]);
+                sacc[pb][0] = acc[0];
+                sacc[pb][1] = acc[1];
+            }
+        } else {
+#pragma unroll
+            for (int pb = 0; pb < 4; ++pb) {
+                const uint32_t row = min(kt * kPrefillTile + 16 * pb + (uint32_t)(l & 15), kv_len - 1);
+                const size_t qr = ((size_t)min(w_t0 + (l & 15), T - 1) * a.q_heads + (size_t)kvh * 2) * kD;
+                f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll 1
+                for (int s = 0; s < 16; ++s) {
+                    const int dim = 32 * (s >> 3) + 8 * (l >> 4) + (s & 7);
+                    const float k = KIo::at(a, kbase, kvh, row, dim);
+#pragma unroll
+                    for (int nt = 0; nt < 2; ++nt)
+                        acc[nt] = mma4(k, load_any(a.query, qr + nt * kD + dim, a.query_dtype), acc[nt]);
+                }
+                sacc[pb][0] = acc[0];
+                sacc[pb][1] = acc[1];
             }
         }
-        // scale, causal mask, online softmax per column
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt) {
-            float tmax = -INFINITY;
+        // causal mask, online softmax per column
+        if ((kt + 1) * kPrefillTile > a.start + w_t0 + 1) {  // some position of the tile is past the first row's
 #pragma unroll
             for (int pb = 0; pb < 4; ++pb)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const uint32_t pos = kt * kPrefillTile + 16 * pb + 4 * lg + j;
-                    const float v = pos <= qpos ? sacc[pb][nt][j] * c : -INFINITY;
-                    sacc[pb][nt][j] = v;
-                    tmax = fmaxf(tmax, v);
+#pragma unroll
+                    for (int nt = 0; nt < 2; ++nt) sacc[pb][nt][j] = pos <= qpos ? sacc[pb][nt][j] : -INFINITY;
                 }
-            tmax = max_xor32(max_xor16(tmax));
-            const float mnew = fmaxf(mrun[nt], tmax);
+        }
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+            float smax = -INFINITY;
+#pragma unroll
+            for (int pb = 0; pb < 4; ++pb)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) smax = fmaxf(smax, sacc[pb][nt][j]);
+            smax = max_xor32(max_xor16(smax));
+            const float mnew = fmaxf(mrun[nt], smax * c);
             const float alpha = fast_exp2(mrun[nt] - mnew);
             mrun[nt] = mnew;
+            const float off = kShift - mnew;
             float ps = 0.0f;
 #pragma unroll
             for (int pb = 0; pb < 4; ++pb)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const float p = fast_exp2(sacc[pb][nt][j] - mnew);
+                    const float p = fast_exp2(__builtin_fmaf(sacc[pb][nt][j], c, off));
                     sacc[pb][nt][j] = p;
                     ps += p;
                 }
@@ -296,30 +456,93 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
             for (int db = 0; db < 4; ++db) oacc[db][nt] *= alpha;
         }
         // O^T += V^T . P^T
+        if (!split) {
 #pragma unroll
-        for (int pb = 0; pb < 4; ++pb)
+            for (int pb = 0; pb < 4; ++pb)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const f32x4 v4 = *reinterpret_cast<const f32x4*>(Vl + (16 * pb + 4 * lg + j) * kRowF + 4 * li);
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t row = min(kt * kPrefillTile + 16 * pb + 4 * (uint32_t)(l >> 4) + j, kv_len - 1);
 #pragma unroll
-                for (int db = 0; db < 4; ++db)
+                    for (int db = 0; db < 4; ++db) {
+                        const float v = VIo::at(a, vbase, kvh, row, 16 * db + (l & 15));
 #pragma unroll
-                    for (int nt = 0; nt < 2; ++nt) oacc[db][nt] = mma4(v4[db], sacc[pb][nt][j], oacc[db][nt]);
+                        for (int nt = 0; nt < 2; ++nt) oacc[db][nt] = mma4(v, sacc[pb][nt][j], oacc[db][nt]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);  // few registers before many loads in flight
+                }
+            return;
+        }
+        const char* vt = st + NK * kPlaneBytes;
+        auto v_operand = [&](int h, int piece, int db) __attribute__((always_inline)) {
+            // rows r and r + 16 share row & 7, so one chunk address serves both
+            const char* p = vt + piece * kPlaneBytes + h * 32 * kD * 2 + plane_chunk(v_row, 2 * db + ((li & 3) >> 1)) +
+                            8 * (li & 1);
+            const i16x4 r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(p));
+            const i16x4 r1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(p + 16 * kD * 2));
+            return __builtin_shufflevector(r0, r1, 0, 1, 2, 3, 4, 5, 6, 7);
+        };
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if constexpr (kHalfV) {
+                f16x8 p0[2], p1[2];
+#pragma unroll
+                for (int nt = 0; nt < 2; ++nt) {
+                    u32x4 w, rest;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const f32x4& s = sacc[2 * h + (e >> 1)][nt];
+                        uint32_t x;
+                        w[e] = round_f16(s[2 * (e & 1)], s[2 * (e & 1) + 1], x);
+                        rest[e] = x;
+                    }
+                    p0[nt] = __builtin_bit_cast(f16x8, w);
+                    p1[nt] = __builtin_bit_cast(f16x8, rest);
+                }
+#pragma unroll
+                for (int db = 0; db < 4; ++db) {
+                    const f16x8 v = __builtin_bit_cast(f16x8, v_operand(h, 0, db));
+#pragma unroll
+                    for (int nt = 0; nt < 2; ++nt) oacc[db][nt] = MfmaT<F16>::mma(v, p1[nt], oacc[db][nt]);
+#pragma unroll
+                    for (int nt = 0; nt < 2; ++nt) oacc[db][nt] = MfmaT<F16>::mma(v, p0[nt], oacc[db][nt]);
+                }
+            } else {
+                u32x4 p[2][3];
+#pragma unroll
+                for (int nt = 0; nt < 2; ++nt) {
+                    float f[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) f[e] = sacc[2 * h + (e >> 2)][nt][e & 3];
+                    split8<3>(f, p[nt]);
+                }
+#pragma unroll
+                for (int db = 0; db < 4; ++db) {
+                    u32x4 v[NV];
+#pragma unroll
+                    for (int i = 0; i < NV; ++i) v[i] = __builtin_bit_cast(u32x4, v_operand(h, i, db));
+#pragma unroll
+                    for (int sum = 2; sum >= 0; --sum)
+#pragma unroll
+                        for (int i = 0; i < NV; ++i)
+#pragma unroll
+                            for (int nt = 0; nt < 2; ++nt)
+                                if (i <= sum) oacc[db][nt] = mma_bf(v[i], p[nt][sum - i], oacc[db][nt]);
+                }
             }
+        }
     };
 
     for (uint32_t r = 0; r < m; ++r) {
-        const int st = (int)(r & 1u);
         const bool more = r + 1 < m;
-        if (more) {  // the next tile's loads are in flight during this tile's math
-            KIo::load(kraw, kbase, t0 + r + 1, kv_len, tid);
-            vload(vraw, t0 + r + 1);
+        if (more) load_tile(t0 + r + 1);  // in flight during this tile's math
+        if (r < wave_m) {
+            const u32x4 w = *reinterpret_cast<const u32x4*>(wide[r & 1]);
+            const bool split = __builtin_amdgcn_readfirstlane(w[0] | w[1] | w[2] | w[3]) == 0;
+            compute(lds[r % STAGES], t0 + r, split);
         }
-        if (r < wave_m) compute(lds[st][0], lds[st][1], t0 + r);
-        if (more) {  // the other stage was last read in round r - 1, before its barrier
-            KIo::store(kraw, lds[st ^ 1][0], tid);
-            vstore(vraw, lds[st ^ 1][1], t0 + r + 1);
-        }
+        if constexpr (STAGES == 1) __syncthreads();
+        // two stages: the other one was last read in round r - 1, before its barrier
+        if (more) store_tile(t0 + r + 1, r + 1);
         __syncthreads();
     }
 
@@ -327,20 +550,18 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
     // the four 16-lane groups hold disjoint positions of each column
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) lsum[nt] = sum_xor32(sum_xor16(lsum[nt]));
-    // lane (g, i) holds dims 16g + 4jj + db of column i as oacc[db][nt][jj]
     if (nchunks > 1) {
         const size_t slot = (((size_t)kvh * nqb + qblock) * a.max_chunks + chunk) * 128;
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
             const size_t colx = slot + wave * 32 + nt * 16 + li;
             if (lg == 0) {
-                a.part_ml[2 * colx] = mrun[nt];
+                a.part_ml[2 * colx] = mrun[nt] - kShift;  // l and O carry the offset
                 a.part_ml[2 * colx + 1] = lsum[nt];
             }
 #pragma unroll
-            for (int jj = 0; jj < 4; ++jj)
-                *reinterpret_cast<f32x4*>(a.part_o + colx * kD + 16 * lg + 4 * jj) =
-                    f32x4{oacc[0][nt][jj], oacc[1][nt][jj], oacc[2][nt][jj], oacc[3][nt][jj]};
+            for (int db = 0; db < 4; ++db)
+                *reinterpret_cast<f32x4*>(a.part_o + colx * kD + 16 * db + 4 * lg) = oacc[db][nt];
         }
         return;
     }
@@ -348,31 +569,33 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
         const float inv = 1.0f / lsum[nt];
-        const size_t obase = ((size_t)tok * a.q_heads + (size_t)kvh * 2 + nt) * kD + 16 * lg;
+        const size_t obase = ((size_t)tok * a.q_heads + (size_t)kvh * 2 + nt) * kD + 4 * lg;
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj)
-#pragma unroll
-            for (int db = 0; db < 4; ++db) store_any(a.out, obase + 4 * jj + db, oacc[db][nt][jj] * inv, a.out_dtype);
+        for (int db = 0; db < 4; ++db) store4_any(a.out, obase + 16 * db, oacc[db][nt] * inv, a.out_dtype);
     }
 }
 
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-// Split KV: a prompt whose query blocks give fewer than kF32TargetWgs
-// workgroups cuts each block's KV range into chunks of at least
-// f32_min_chunk_tiles tiles.  The kernel is bound by the fp32 matrix cores
-// (a 64-position tile is about 4 us of one wave's matrix-core time), so the
-// longest block's chain of tiles sets the time unless it is cut short.
-// Measured, Granite 2048-token prompt at start 0 (Fp32KFp16V / fp32 K/V, us):
-// 512 workgroups and chunks of 8 tiles or more 160 / 159, 1024 and 4 tiles
-// 129 / 128, 1024 and 2 tiles 130 / 127, 2048 and 4 tiles 119.5 / 117.5.
-// Floors of 4 / 2 / 1 tiles, Fp32KFp16V (us per prefill, start + T): 0 + 128
-// 16.3 / 16.2 / 14.4, 0 + 256 25.4 / 19.6 / 15.7, 0 + 512 31.0 / 23.3 / 25.3,
-// 0 + 1024 51.7 / 49.3 / 54.6, 1000 + 100 30.7 / 20.3 / 24.3, 2048 tokens and
-// more the same: one tile for prompts of at most four, two otherwise.
-constexpr uint32_t kF32TargetWgs = 2048;
-static uint32_t f32_min_chunk_tiles(uint32_t n_max) { return n_max <= 4 ? 1u : 2u; }
+// Split KV.  A workgroup costs about 5 us beside its tiles (query pieces,
+// first tile, partials) and a tile about 3.2 us where two workgroups share a
+// CU, so a block's KV range is cut
+// - into enough chunks for kF32TargetWgs workgroups (two per CU), each at
+//   least kF32MinTiles tiles, and
+// - into chunks of about kF32ChunkTiles tiles while that makes at most
+//   kF32MostWgs workgroups: with more blocks than CUs the longest block's
+//   chain would set the time.
+// Measured, Fp32KFp16V, us per layer of an 8-layer prompt (front end and
+// merge included), start + T: at least 8 tiles a chunk / this rule 0 + 256
+// 21.2 / 20.0, 0 + 512 30.9 / 23.3, 1000 + 100 35.5 / 22.8, 2000 + 500 47.5 /
+// 41.4; toward 512 workgroups only / this rule 0 + 3000 111.0 / 104.9; toward
+// 2048 with 2 tiles (the fp32 matrix cores' rule) / this rule 2000 + 500
+// 49.0 / 41.4, 0 + 3000 110.0 / 104.9, 0 + 1900 60.5 / 60.0.
+constexpr uint32_t kF32TargetWgs = 512;
+constexpr uint32_t kF32MinTiles = 2;
+constexpr uint32_t kF32ChunkTiles = 8;
+constexpr uint32_t kF32MostWgs = 2048;
 constexpr uint32_t kF32MaxChunks = 32;
 constexpr uint32_t kF32Columns = 128;
 
@@ -388,24 +611,23 @@ static uint32_t f32_blocks(const ShapeDims& s, uint32_t tokens) {
     return (tokens + kPrefillTile - 1) / kPrefillTile * s.kv_heads;
 }
 
-// most chunks a block can take in a cache of `capacity` positions
-static uint32_t f32_max_chunks(const ShapeDims& s, uint32_t tokens, uint32_t capacity) {
+// chunks of a block of `tiles` tiles
+static uint32_t f32_chunks(const ShapeDims& s, uint32_t tokens, uint32_t tiles) {
     const uint32_t wgs = f32_blocks(s, tokens);
-    if (wgs >= kF32TargetWgs) return 1;
-    uint32_t want = (kF32TargetWgs + wgs - 1) / wgs;
-    if (want > kF32MaxChunks) want = kF32MaxChunks;
-    const uint32_t fit = (capacity + kPrefillTile - 1) / kPrefillTile;  // the one-tile floor
-    if (want > fit) want = fit;
-    return want < 1 ? 1 : want;
+    const uint32_t fill = std::min((kF32TargetWgs + wgs - 1) / wgs, tiles / kF32MinTiles);
+    const uint32_t cut = std::min(kF32MostWgs / wgs, tiles / kF32ChunkTiles);
+    return std::max(1u, std::min(kF32MaxChunks, std::max(fill, cut)));
 }
 
-static uint32_t f32_chunk_tiles(const ShapeDims& s, uint32_t start, uint32_t tokens, uint32_t capacity) {
-    const uint32_t want = f32_max_chunks(s, tokens, capacity);
+// most chunks a block can take in a cache of `capacity` positions
+static uint32_t f32_max_chunks(const ShapeDims& s, uint32_t tokens, uint32_t capacity) {
+    return f32_chunks(s, tokens, (capacity + kPrefillTile - 1) / kPrefillTile);
+}
+
+static uint32_t f32_chunk_tiles(const ShapeDims& s, uint32_t start, uint32_t tokens) {
     const uint32_t n_max = (start + tokens + kPrefillTile - 1) / kPrefillTile;
-    const uint32_t fit = n_max / f32_min_chunk_tiles(n_max);
-    const uint32_t chunks = want < fit ? want : fit;
-    if (chunks <= 1) return 0;
-    return (n_max + chunks - 1) / chunks;
+    const uint32_t chunks = f32_chunks(s, tokens, n_max);
+    return chunks <= 1 ? 0 : (n_max + chunks - 1) / chunks;
 }
 
 uint64_t prefill_f32_workspace_bytes(const ShapeDims& s, uint32_t capacity, uint32_t tokens) {
@@ -441,7 +663,7 @@ hipError_t launch_prefill_f32(const ShapeDims& s, const KvLayer& kv, uint32_t st
     a.kv_heads = s.kv_heads;
     a.qblocks = (tokens + kPrefillTile - 1) / kPrefillTile;
     a.xcd_map = (8 % s.kv_heads == 0) && ((uint64_t)a.qblocks * s.kv_heads) % 8 == 0;
-    a.chunk_tiles = f32_chunk_tiles(s, start, tokens, kv.capacity);
+    a.chunk_tiles = f32_chunk_tiles(s, start, tokens);
     a.max_chunks = f32_max_chunks(s, tokens, kv.capacity);
     const uint64_t slots = (uint64_t)a.qblocks * s.kv_heads * a.max_chunks * kF32Columns;
     a.part_ml = reinterpret_cast<float*>(workspace);

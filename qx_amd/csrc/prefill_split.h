@@ -136,8 +136,7 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillPipeArgs a)
     }
     const float inv = 1.0f / L;
     const size_t obase = ((size_t)tok * a.q_heads + head) * D + 4 * d4;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) store_any(a.out, obase + j, O[j] * inv, a.out_dtype);
+    store4_any(a.out, obase, O * inv, a.out_dtype);
 }
 
 }  // namespace qxh
