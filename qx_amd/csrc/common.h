@@ -86,6 +86,13 @@ template <bool NT> __device__ __forceinline__ u32x4 load16(const void* p) {
     else return *q;
 }
 
+// 16 bytes from an address with the element's own alignment only (caller
+// buffers whose alignment no entry point asks for).
+typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ u32x4 load16_any(const uint16_t* p) { return *reinterpret_cast<const u32x4_a2*>(p); }
+__device__ __forceinline__ u32x4 load16_any(const float* p) { return *reinterpret_cast<const u32x4_a4*>(p); }
+
 // Unpack the 16 bytes of a row slice into EPL floats.
 template <int DT> struct Unpack;
 template <> struct Unpack<F32> {
