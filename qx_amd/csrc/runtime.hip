@@ -107,8 +107,16 @@ static uint64_t align256(uint64_t x) { return (x + 255) & ~(uint64_t)255; }
 
 // Qwen RoPE inverse frequencies formed exactly as the reference CPU path does,
 // 1e6_f32.powf(-(i as f32) / 64.0) (tools/qx-qwen-parity/src/main.rs:1193).
+// Formed once: 64 powf cost an encode more than its launch.
 static void qwen_inverse_frequencies(float* out) {
-    for (int i = 0; i < 64; ++i) out[i] = powf(1000000.0f, -(float)i / 64.0f);
+    struct Table {
+        float f[64];
+        Table() {
+            for (int i = 0; i < 64; ++i) f[i] = powf(1000000.0f, -(float)i / 64.0f);
+        }
+    };
+    static const Table table;  // initialised once, whichever thread comes first
+    memcpy(out, table.f, sizeof table.f);
 }
 
 // ---------------------------------------------------------------------------

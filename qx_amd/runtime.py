@@ -40,7 +40,7 @@ def _ptr(t):
         raise ValueError("tensor must live on the GPU")
     if not t.is_contiguous():
         raise ValueError("tensor must be contiguous")
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()  # a plain int: the argtypes make it a pointer
 
 
 def shape_info(shape: int) -> abi.ShapeInfo:
@@ -170,6 +170,8 @@ class KvArena:
                                         nbytes.value, ctypes.byref(h)))
         self._h = h
         self.info = shape_info(shape)
+        # plain ints for the encoders, which check every call's shapes against them
+        self._heads = (self.info.q_heads, self.info.kv_heads, self.info.head_dim)
         self.layout = abi.KvLayout()
         check(lib().qxh_kv_cache_layout(self._h, ctypes.byref(self.layout)))
 
@@ -261,13 +263,15 @@ def rope_kv_batch(graph: Graph, cache: KvArena, layer: int, start_position: int,
 
     key/value: [sequences][tokens][kv_heads][d]; query/query_out:
     [sequences][tokens][q_heads][d] (query_out may be None)."""
-    kvh, d = cache.info.kv_heads, cache.info.head_dim
-    seqs, tokens = key.shape[0], key.shape[1]
-    if key.shape[2:] != (kvh, d) or value.shape != key.shape:
+    qh, kvh, d = cache._heads
+    shape = key.shape
+    seqs, tokens = shape[0], shape[1]
+    if shape != (seqs, tokens, kvh, d) or value.shape != shape:
         raise ValueError(f"key/value must be [S][T][{kvh}][{d}], got {tuple(key.shape)} / {tuple(value.shape)}")
-    if query is not None and query.shape != (seqs, tokens, cache.info.q_heads, d):
-        raise ValueError(f"query must be [S][T][{cache.info.q_heads}][{d}], got {tuple(query.shape)}")
-    if query_out is not None and query_out.shape != (seqs, tokens, cache.info.q_heads, d):
+    wanted = (seqs, tokens, qh, d)
+    if query is not None and query.shape != wanted:
+        raise ValueError(f"query must be [S][T][{qh}][{d}], got {tuple(query.shape)}")
+    if query_out is not None and query_out.shape != wanted:
         raise ValueError("query_out shape mismatch")
     dt = qxh_dtype(key)
     if value.dtype != key.dtype or (query is not None and query.dtype != key.dtype):
@@ -303,14 +307,14 @@ def decode_step(graph: Graph, cache: KvArena, layer: int, position: int, query, 
     """RoPE + append + attention of one Granite token (fp32 q [16][64], k/v [8][64])
     for sequence 0 over positions [0, position]; returns out [16][64]."""
     if out is None:
-        out = torch.empty((cache.info.q_heads, cache.info.head_dim), dtype=out_dtype or torch.float32,
+        out = torch.empty((cache._heads[0], cache._heads[2]), dtype=out_dtype or torch.float32,
                           device=query.device)
     ws_bytes = 0
     if workspace is None and (position + 1 > 1024 or cache.value_dtype == abi.I8_TIERED):  # the two-call path
         need = attention_workspace_bytes(cache, 1, position + 1)
         workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=query.device) if need else None
     if workspace is not None:
-        ws_bytes = workspace.numel() * workspace.element_size()
+        ws_bytes = workspace.nbytes
     check(lib().qxh_encode_decode_step_for_layer(graph.handle, cache.handle, _ptr(query), _ptr(key), _ptr(value),
                                                  _ptr(query_out), layer, position, _ptr(out), qxh_dtype(out),
                                                  _ptr(workspace), ws_bytes))
@@ -322,15 +326,18 @@ def attention(graph: Graph, cache: KvArena, layer: int, query, length: int, out=
     """Decode attention of one query token per sequence over positions [0, length).
 
     query: [sequences][q_heads][d]; returns out of the same shape."""
-    seqs = query.shape[0]
-    if query.shape[1:] != (cache.info.q_heads, cache.info.head_dim):
-        raise ValueError(f"query must be [S][{cache.info.q_heads}][{cache.info.head_dim}]")
+    qh, _, d = cache._heads
+    shape = query.shape
+    seqs = shape[0]
+    if shape != (seqs, qh, d):
+        raise ValueError(f"query must be [S][{qh}][{d}]")
     if out is None:
-        out = torch.empty(query.shape, dtype=out_dtype or query.dtype, device=query.device)
-    need = attention_workspace_bytes(cache, seqs, length)
-    if workspace is None and need:
-        workspace = torch.empty(need, dtype=torch.uint8, device=query.device)
-    ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
+        out = torch.empty(shape, dtype=out_dtype or query.dtype, device=query.device)
+    if workspace is None:  # a given one is checked by the encoder
+        need = attention_workspace_bytes(cache, seqs, length)
+        if need:
+            workspace = torch.empty(need, dtype=torch.uint8, device=query.device)
+    ws_bytes = workspace.nbytes if workspace is not None else 0
     check(lib().qxh_encode_attention_for_layer(graph.handle, cache.handle, layer, first_sequence, seqs, length,
                                                _ptr(query), qxh_dtype(query), _ptr(out), qxh_dtype(out),
                                                _ptr(workspace), ws_bytes))
@@ -362,10 +369,11 @@ def prefill_attention(graph: Graph, cache: KvArena, layer: int, start_position: 
     tokens = query.shape[0]
     if out is None:
         out = torch.empty(query.shape, dtype=out_dtype or query.dtype, device=query.device)
-    need = prefill_workspace_bytes(cache, tokens)
-    if workspace is None and need:
-        workspace = torch.empty(need, dtype=torch.uint8, device=query.device)
-    ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
+    if workspace is None:  # a given one is checked by the encoder
+        need = prefill_workspace_bytes(cache, tokens)
+        if need:
+            workspace = torch.empty(need, dtype=torch.uint8, device=query.device)
+    ws_bytes = workspace.nbytes if workspace is not None else 0
     check(lib().qxh_encode_prefill_attention(graph.handle, cache.handle, layer, sequence, start_position, tokens,
                                              _ptr(query), qxh_dtype(query), _ptr(out), qxh_dtype(out),
                                              _ptr(workspace), ws_bytes))
