@@ -24,6 +24,7 @@
 #include "mfma.h"
 #include "tiered_v.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace qxh {
@@ -1002,6 +1003,225 @@ __global__ __launch_bounds__(64 * WAVES) void decode_mfma_kernel(DecodeArgs a) {
     decode_mfma_body<D, G, KDT, WAVES, TV, false>(a, nullptr);
 }
 
+// ---------------------------------------------------------------------------
+// Causal rows of one sequence on the matrix cores (equal 16-bit caches): the
+// few-row prefill calls, a drafted block to verify.  A row attends all cached
+// positions but the last few, so a workgroup takes 16 / G rows at once,
+// their G heads each as the 16 columns of S^T, and streams its range of the
+// K/V rows once for all of them (decode_mfma_kernel, one row a workgroup,
+// streams it once per row and leaves 16 - G columns idle).  Tiles, operands and
+// the two register sets are decode_mfma_body's; column (row t, head g) masks
+// positions past causal_start + t.  The partials are decode_combine_kernel's.
+// Bound by the K/V rows' round trips and the merge: 8 Qwen rows over 30000
+// positions (61 MB a layer) 29.4 us, 44.6 with a row a workgroup; 8 Granite
+// rows over 3900 8.2 against 10.6.
+// ---------------------------------------------------------------------------
+template <int D, int G, int KDT>
+__global__ __launch_bounds__(256) void decode_mfma_rows_kernel(DecodeArgs a) {
+    using M = MfmaT<KDT>;
+    using vec = typename M::vec;
+    constexpr int WAVES = 4;
+    constexpr int KSTEPS = D / 32, DTILES = D / 16;
+    constexpr int VROWB = D * 2 + 32;
+    constexpr int VCH = 32 * D * 2 / 16 / 64;
+    constexpr uint32_t ROWS = 16 / G;
+    __shared__ __attribute__((aligned(16))) char vtile[WAVES][32 * VROWB];
+    __shared__ float sm_m[WAVES][16], sm_l[WAVES][16];
+    __shared__ __attribute__((aligned(16))) float sm_acc[WAVES][16][D];
+
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int lg = lane >> 4, li = lane & 15;
+    const uint32_t split = blockIdx.x, kvh = blockIdx.y, hkv = gridDim.y;
+    const uint32_t T = a.length - a.causal_start;
+    const uint32_t t0 = blockIdx.z * ROWS;  // this workgroup's first row
+    const uint32_t r0 = split * a.chunk;
+    const uint32_t r1 = min(min(a.length, a.causal_start + t0 + ROWS), r0 + a.chunk);
+    const float c = a.qscale;
+    char* vl = vtile[wave];
+    const uint32_t common = a.causal_start + t0 + 1;  // positions every row of the workgroup attends
+    const uint16_t* vhead = reinterpret_cast<const uint16_t*>(a.values) + (size_t)kvh * a.head_stride;
+
+    // column li: row t0 + li / G, head li % G
+    const uint32_t limit = min(r1, common + li / G);  // positions the column attends
+    vec qop[KSTEPS];
+    float mrun = kNegBig, lrun = 0.f;
+    f32x4 oacc[DTILES];
+#pragma unroll
+    for (int dt = 0; dt < DTILES; ++dt) oacc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto load_q = [&]() __attribute__((always_inline)) {
+        const uint32_t row = min(t0 + li / G, T - 1);  // past the call: computed, never stored
+        const size_t q0 = (((size_t)row * hkv + kvh) * G + li % G) * D;
+        if (a.query_dtype == KDT) {
+#pragma unroll
+            for (int ks = 0; ks < KSTEPS; ++ks)
+                qop[ks] = __builtin_bit_cast(vec, load16<false>(reinterpret_cast<const char*>(a.query) +
+                                                                (q0 + 32 * ks + 8 * lg) * 2));
+        } else {
+#pragma unroll
+            for (int ks = 0; ks < KSTEPS; ++ks)
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    qop[ks][j] = M::cvt(load_any(a.query, q0 + 32 * ks + 8 * lg + j, a.query_dtype));
+        }
+    };
+    auto compute = [&](uint32_t base, const u32x4 (&kr)[2][KSTEPS], const u32x4 (&vr)[VCH])
+                       __attribute__((always_inline)) {
+        // A later row's value may be infinite: its zero probability in an
+        // earlier row's column would make that row NaN, so such a tile keeps
+        // the rows past `common` out of the matrix product.
+        bool apart = false;
+        if (base + 32 > common) {
+#pragma unroll
+            for (int cc = 0; cc < VCH; ++cc) {
+                constexpr uint32_t kExp = KDT == F16 ? 0x7c00u : 0x7f80u;
+                if (base + (lane + 64 * cc) / (D / 8) >= common)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        apart |= (vr[cc][j] & kExp) == kExp || ((vr[cc][j] >> 16) & kExp) == kExp;
+            }
+            apart = __any(apart);
+        }
+#pragma unroll
+        for (int cc = 0; cc < VCH; ++cc) {
+            const int chunk = lane + 64 * cc;
+            const bool out = apart && base + chunk / (D / 8) >= common;
+            *reinterpret_cast<u32x4*>(vl + chunk / (D / 8) * VROWB + chunk % (D / 8) * 16) =
+                out ? u32x4{0u, 0u, 0u, 0u} : vr[cc];
+        }
+        f32x4 sacc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks)
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt) sacc[mt] = M::mma(__builtin_bit_cast(vec, kr[mt][ks]), qop[ks], sacc[mt]);
+        float sv[8];
+        float tmax = -INFINITY;
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t pos = base + 16 * mt + 4 * lg + j;
+                const float v = pos < limit ? sacc[mt][j] * c : -INFINITY;
+                sv[mt * 4 + j] = v;
+                tmax = fmaxf(tmax, v);
+            }
+        tmax = max_xor32(max_xor16(tmax));
+        const float mnew = fmaxf(mrun, tmax);
+        const float alpha = fast_exp2(mrun - mnew);
+        mrun = mnew;
+        vec phi, plo;
+        float psum = 0.f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const float p = fast_exp2(sv[k] - mnew);
+            psum += p;
+            const auto h = M::cvt(p);
+            phi[k] = h;
+            if constexpr (KDT == BF16) plo[k] = M::cvt(p - (float)h);
+        }
+        lrun = __builtin_fmaf(lrun, alpha, psum);
+#pragma unroll
+        for (int dt = 0; dt < DTILES; ++dt) oacc[dt] *= alpha;
+        if (apart) {
+            // the rows past `common` one by one, straight from the cache: lane
+            // (g, i) adds to its own dims of column i where the column attends
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                float p = (float)phi[k];
+                if constexpr (KDT == BF16) p += (float)plo[k];
+#pragma unroll 1
+                for (int g = 0; g < 4; ++g) {
+                    const uint32_t pos = base + 16 * (k >> 2) + 4 * g + (k & 3);
+                    const float pg = __shfl(p, 16 * g + li);
+                    if (pos < common || pos >= limit) continue;
+#pragma unroll
+                    for (int dt = 0; dt < DTILES; ++dt)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const uint16_t v = vhead[(size_t)pos * D + 16 * dt + 4 * lg + j];
+                            oacc[dt][j] = __builtin_fmaf(pg, KDT == F16 ? half_bits_to_f32(v) : bf16_to_f32(v), oacc[dt][j]);
+                        }
+                }
+            }
+        }
+#pragma unroll
+        for (int dt = 0; dt < DTILES; ++dt) {
+            const vec vop = __builtin_bit_cast(vec, vt_operand_rows32<VROWB>(vl, 0, 16 * dt, lg, li));
+            oacc[dt] = M::mma(vop, phi, oacc[dt]);
+            if constexpr (KDT == BF16) oacc[dt] = M::mma(vop, plo, oacc[dt]);
+        }
+    };
+
+    if (r1 > r0) {
+        const char* kb = reinterpret_cast<const char*>(a.keys) + ((size_t)kvh * a.head_stride + (size_t)r0 * D) * 2;
+        const char* vb = reinterpret_cast<const char*>(a.values) + ((size_t)kvh * a.head_stride + (size_t)r0 * D) * 2;
+        const __amdgpu_buffer_rsrc_t krs = dec_rsrc(kb, (r1 - r0) * D * 2), vrs = dec_rsrc(vb, (r1 - r0) * D * 2);
+        auto bload_tile = [&](uint32_t t, u32x4 (&kr)[2][KSTEPS], u32x4 (&vr)[VCH]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+                for (int ks = 0; ks < KSTEPS; ++ks)
+                    kr[mt][ks] = bload16<false>(krs, ((t * 32 + 16 * mt + li) * D + 32 * ks + 8 * lg) * 2);
+#pragma unroll
+            for (int cc = 0; cc < VCH; ++cc) {
+                const int chunk = lane + 64 * cc;
+                vr[cc] = bload16<true>(vrs, ((t * 32 + chunk / (D / 8)) * D + (chunk % (D / 8)) * 8) * 2);
+            }
+        };
+        const uint32_t ntiles = (r1 - r0 + 31) / 32;
+        const uint32_t n = ntiles > (uint32_t)wave ? (ntiles - wave + WAVES - 1) / WAVES : 0u;
+        if (n > 0) {
+            u32x4 kr0[2][KSTEPS], vr0[VCH], kr1[2][KSTEPS], vr1[VCH];
+            bload_tile(wave, kr0, vr0);
+            load_q();
+            for (uint32_t j = 0; j < n; j += 2) {
+                const uint32_t t = wave + j * WAVES;
+                bload_tile(t + WAVES, kr1, vr1);
+                __builtin_amdgcn_sched_barrier(0);  // the prefetch goes out before this tile's math
+                compute(r0 + 32 * t, kr0, vr0);
+                bload_tile(t + 2 * WAVES, kr0, vr0);
+                __builtin_amdgcn_sched_barrier(0);
+                if (j + 1 < n) compute(r0 + 32 * (t + WAVES), kr1, vr1);
+            }
+        }
+    }
+
+    // merge the waves: a thread owns four dims of a column at a time
+    lrun = sum_xor32(sum_xor16(lrun));
+#pragma unroll
+    for (int dt = 0; dt < DTILES; ++dt) *reinterpret_cast<f32x4*>(&sm_acc[wave][li][16 * dt + 4 * lg]) = oacc[dt];
+    if (lg == 0) {
+        sm_m[wave][li] = mrun;
+        sm_l[wave][li] = lrun;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = threadIdx.x; i < 16 * D / 4; i += 64 * WAVES) {
+        const int col = i / (D / 4), d = 4 * (i % (D / 4));
+        const uint32_t row = t0 + col / G, g = col % G;
+        if (row >= T) continue;
+        float Mx = kNegBig;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) Mx = fmaxf(Mx, sm_m[w][col]);
+        float L = 0.0f;
+        f32x4 A = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            const float f = fast_exp2(sm_m[w][col] - Mx);
+            L = __builtin_fmaf(sm_l[w][col], f, L);
+            const f32x4 v = *reinterpret_cast<const f32x4*>(&sm_acc[w][col][d]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) A[j] = __builtin_fmaf(v[j], f, A[j]);
+        }
+        if (a.splits == 1) {
+            store4_any(a.out, (((size_t)row * hkv + kvh) * G + g) * D + d, A * (1.0f / L), a.out_dtype);
+        } else {
+            const size_t p = (((size_t)row * hkv + kvh) * a.splits + split) * G + g;
+            *reinterpret_cast<f32x4*>(a.ws_acc + p * D + d) = A;
+            if (d == 0) *reinterpret_cast<float2*>(a.ws_ml + 2 * p) = float2{Mx, L};
+        }
+    }
+}
+
 // The Qwen block's decode with its front end folded in (QwenFrontArgs).
 template <int KDT>
 __global__ __launch_bounds__(256) void decode_mfma_front_kernel(DecodeArgs a, QwenFrontArgs f) {
@@ -1496,7 +1716,69 @@ hipError_t launch_block_decode_attention(const ShapeDims& s, const KvLayer& kv, 
     return hipGetLastError();
 }
 
+// Causal rows of equal 16-bit caches: 16 / group of them to a workgroup
+// (decode_mfma_rows_kernel) where streaming the K/V rows once for all of them
+// outweighs the wider merge, one a workgroup (decode_mfma_kernel, which keeps
+// short contexts in one chunk) below.  Measured, us per call with the KV from
+// HBM (one row a workgroup / several, start + rows):
+// - Qwen bf16 4000 + 3 10.0 / 10.5, 8000 + 3 13.2 / 12.5, 2000 + 8 10.2 /
+//   10.8, 4000 + 8 12.5 / 12.2, 12000 + 5 18.9 / 17.7, 30000 + 8 44.6 / 29.4,
+//   4000 + 16 17.9 / 14.7; past 32 rows one a workgroup makes a single round
+//   of the CUs and no merge: 2000 + 48 23.1 / 22.7, 2000 + 63 23.8 / 25.5,
+//   4000 + 48 40.3 / 31.6;
+// - Granite f16 1200 + 5 6.8 / 7.4, 2000 + 5 7.5 / 7.4, 3900 + 8 10.6 / 8.2,
+//   800 + 12 8.1 / 7.5, 800 + 24 6.7 / 7.8 (one chunk from 16 to 32 rows),
+//   1200 + 24 8.6 / 8.1, 3900 + 24 20.6 / 9.6, 500 + 48 8.0 / 8.0, 800 + 48
+//   10.8 / 8.5.
+static bool rows_on_mfma(const ShapeDims& s, int key_dtype, int value_dtype, uint32_t start, uint32_t tokens) {
+    if (key_dtype != value_dtype || (key_dtype != F16 && key_dtype != BF16) || tokens < 2) return false;
+    const uint64_t length = (uint64_t)start + tokens, pairs = tokens * length;
+    if (s.group >= 8) return tokens <= 32 ? pairs >= 20000 : length >= 2560;
+    return pairs >= 11000 && length > (tokens >= 16 && tokens <= 32 ? 1152u : 640u);
+}
+
+static DecodePlan plan_rows_mfma(const ShapeDims& s, uint32_t start, uint32_t tokens) {
+    DecodePlan p{};
+    p.waves = kWaves;
+    const uint32_t per = 16 / (uint32_t)s.group, length = start + tokens;
+    const uint32_t units = (uint32_t)s.kv_heads * ((tokens + per - 1) / per);
+    // one workgroup a CU, of at least a tile a wave: 192 and 384 workgroups,
+    // and splits of 256 positions, measured the same or slower (Qwen 12000 +
+    // 8, 192 / 256 / 384 workgroups 20.0 / 17.8 / 24.0 us)
+    const uint32_t gran = kWaves * 32;
+    const uint32_t splits = std::max(1u, std::min(kDecodeCus / units, (length + gran - 1) / gran));
+    p.chunk = ((length + splits - 1) / splits + gran - 1) / gran * gran;
+    p.splits = (length + p.chunk - 1) / p.chunk;
+    p.workspace_bytes =
+        p.splits > 1 ? (uint64_t)tokens * s.kv_heads * p.splits * s.group * (s.head_dim + 2) * sizeof(float) : 0;
+    return p;
+}
+
+static hipError_t launch_rows_mfma(const ShapeDims& s, const KvLayer& kv, const DecodePlan& p, DecodeArgs& a,
+                                   uint32_t tokens, void* workspace, hipStream_t st, int* dispatches) {
+    if (p.splits > 1) {
+        a.ws_ml = reinterpret_cast<float*>(workspace);
+        a.ws_acc = a.ws_ml + 2 * (uint64_t)tokens * s.kv_heads * p.splits * s.group;
+    }
+    const uint32_t per = 16 / (uint32_t)s.group;
+    const dim3 grid(p.splits, s.kv_heads, (tokens + per - 1) / per), block(64 * kWaves);
+    const bool granite = s.head_dim == 64 && s.group == 2, f16 = kv.key_dtype == F16;
+    if (granite && f16) hipLaunchKernelGGL((decode_mfma_rows_kernel<64, 2, F16>), grid, block, 0, st, a);
+    else if (granite) hipLaunchKernelGGL((decode_mfma_rows_kernel<64, 2, BF16>), grid, block, 0, st, a);
+    else if (f16) hipLaunchKernelGGL((decode_mfma_rows_kernel<128, 8, F16>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((decode_mfma_rows_kernel<128, 8, BF16>), grid, block, 0, st, a);
+    *dispatches = 1;
+    if (p.splits > 1) {
+        const dim3 cgrid(s.q_heads * (s.head_dim / kCombineDims), tokens);
+        if (granite) hipLaunchKernelGGL((decode_combine_kernel<64, 2>), cgrid, dim3(kCombineThreads), 0, st, a);
+        else hipLaunchKernelGGL((decode_combine_kernel<128, 8>), cgrid, dim3(kCombineThreads), 0, st, a);
+        *dispatches = 2;
+    }
+    return hipGetLastError();
+}
+
 DecodePlan plan_decode_causal(const ShapeDims& s, int key_dtype, int value_dtype, uint32_t start, uint32_t tokens) {
+    if (rows_on_mfma(s, key_dtype, value_dtype, start, tokens)) return plan_rows_mfma(s, start, tokens);
     return plan_decode(s, key_dtype, value_dtype, tokens, start + tokens);
 }
 
@@ -1530,6 +1812,8 @@ hipError_t launch_decode_causal_rows(const ShapeDims& s, const KvLayer& kv, cons
     a.ring_seq_stride = 0;
     a.causal = 1;
     a.causal_start = start;
+    if (rows_on_mfma(s, kv.key_dtype, kv.value_dtype, start, tokens))
+        return launch_rows_mfma(s, kv, p, a, tokens, workspace, st, dispatches);
     return launch_decode_impl(s, kv, p, a, tokens, workspace, st, dispatches);
 }
 

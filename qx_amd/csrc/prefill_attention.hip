@@ -37,19 +37,17 @@ constexpr uint32_t kExactPassWgs = 256;
 // Qwen bf16 at 1020 cached positions 14 / 31 for 1-8 rows, 31 / 32 for 63;
 // at 8188, 42 / 56 for 16 rows; at 32764, 19 / 71 for one row, 71 / 71 for 8,
 // 142 / 69 for 16.  Granite f16 at 3840: 18 / 17 for 16 rows, 48 / 20 for 63.
-// Rows run on the decode kernels up to 8 of them, or, below 64, while
-// (rows - c) x context stays under the crossover measured against the kernel
-// the call would take otherwise (rows / tiled, us, 9-63 rows over 0-32000
-// cached positions, each case timed both ways in one process):
-// - Qwen (c = 6, 126000): 4000 + 32 29.0 / 38.7, 4000 + 48 41.0 / 34.1,
-//   16000 + 12 40.2 / 43.9, 16000 + 16 45.4 / 43.8, 32000 + 9 53.2 / 59.3,
-//   32000 + 12 69.3 / 59.3;
-// - Granite f16 (c = 0, 70000, and at least 64 cached positions; the
-//   pipelined kernel reads V straight from the cache, one dispatch):
-//   2000 + 32 12.1 / 13.2, 1500 + 48 17.2 / 14.4, 4000 + 9 12.2 / 13.7,
-//   4000 + 12 15.4 / 13.7, 0 + 9 7.7 / 5.9;
-// - Granite bf16 (c = 0, 90000): 3000 + 32 17.1 / 19.1, 2000 + 48 21.7 /
-//   18.2, 8000 + 9 18.5 / 24.5, 8000 + 16 25.3 / 24.2;
+// Rows run on the decode kernels up to 8 of them, or, below 64, while rows x
+// context stays under the crossover measured against the kernel the call would
+// take otherwise (rows / tiled, us, 9-63 rows over 64-30000 cached positions,
+// each case timed both ways in one process; several rows share a workgroup,
+// decode_mfma_rows_kernel):
+// - Qwen (450000 up to 32 rows, 300000 beyond): 30000 + 12 39.5 / 64.1, 30000
+//   + 24 69.8 / 64.3, 16000 + 24 43.6 / 49.1, 16000 + 32 49.7 / 49.3, 8000 +
+//   32 31.0 / 43.9, 4000 + 63 33.7 / 37.8, 8000 + 48 50.4 / 43.6;
+// - Granite f16 (500000, and at least 64 cached positions) and bf16 (500000):
+//   the rows win over the whole range, f16 250 + 9 3.9 / 8.7, 2000 + 48 9.9 /
+//   14.6, 3900 + 63 12.6 / 19.5, bf16 3900 + 63 13.2 / 22.3;
 // - the Granite split-product kernel (fp32 and mixed caches; c = 0, 22000):
 //   Fp32KFp16V 1000 + 16 10.4 / 11.0, 500 + 32 12.1 / 12.9, 2000 + 9 13.6 /
 //   12.3, 1000 + 24 14.1 / 11.4, 500 + 48 14.4 / 13.2; fp32 K/V 500 + 48
@@ -67,10 +65,10 @@ static bool rows_on_decode(const ShapeDims& s, int key_dtype, int value_dtype, u
     if (tokens >= 64) return false;
     const uint64_t length = (uint64_t)start + tokens;
     if (s.group >= 8)
-        return value_dtype == I8T ? tokens * length <= 150000u : (tokens - 6) * length <= 126000u;
+        return tokens * length <= (value_dtype == I8T ? 150000u : tokens <= 32 ? 450000u : 300000u);
     if (prefill_f32_supported(s, key_dtype, value_dtype)) return tokens * length <= 22000u;
-    if (key_dtype == F16 && value_dtype == F16) return start >= 64 && tokens * length <= 70000u;
-    if (key_dtype == BF16 && value_dtype == BF16) return tokens * length <= 90000u;
+    if (key_dtype == F16 && value_dtype == F16) return start >= 64 && tokens * length <= 500000u;
+    if (key_dtype == BF16 && value_dtype == BF16) return tokens * length <= 500000u;
     return tokens * length <= 40000u;
 }
 

@@ -1,0 +1,77 @@
+"""Few causal rows over equal 16-bit caches (a drafted block to verify, a short
+chunk of a prompt), where several rows share a workgroup
+(decode_mfma_rows_kernel): row counts around a workgroup's rows (two on the
+Qwen shape, eight on Granite's), contexts around the rules' lines and the
+split's granularity of 128, against float64 attention over the cache's rows at
+the 16-bit bar; and an infinite value in a later drafted row, which must not
+reach the rows before it."""
+import numpy as np
+import pytest
+import torch
+
+from qx_amd import abi
+from qx_amd import runtime as rt
+from tests.helpers import TOL_16, attend64, log, rel_err
+
+pytestmark = pytest.mark.gpu
+
+TORCH = {abi.F32: torch.float32, abi.F16: torch.float16, abi.BF16: torch.bfloat16}
+HEADS = {abi.SHAPE_GRANITE: (16, 8, 64, 0.015625), abi.SHAPE_QWEN3: (32, 4, 128, 128.0 ** -0.5)}
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    return rt.Context(0)
+
+
+def rows(ctx, shape, dt, start, T, seed, plant=None):
+    hq, hk, d, scale = HEADS[shape]
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    arena = rt.KvArena(ctx, shape, 1, 1, start + T, dt)
+    k = torch.randn((1, start + T, hk, d), generator=g, device="cuda").to(TORCH[dt])
+    v = torch.randn((1, start + T, hk, d), generator=g, device="cuda").to(TORCH[dt])
+    if plant is not None:
+        v[0, start + plant[0], plant[1], plant[2]] = float("inf")
+    q = (2 * torch.randn((T, hq, d), generator=g, device="cuda")).to(TORCH[dt])
+    with rt.Graph(ctx) as graph:
+        rt.store_kv(graph, arena, 0, 0, k, v)
+        out = rt.prefill_attention(graph, arena, 0, start, q, out_dtype=torch.float32)
+    return [x.float().cpu().numpy() for x in (q, k[0], v[0], out)]
+
+
+CASES = [(abi.SHAPE_QWEN3, s, T) for s, T in ((9999, 2), (6700, 3), (4091, 5), (2490, 8), (2220, 9), (1250, 17),
+                                              (640, 32), (2528, 33), (2500, 63), (100, 63), (3000, 2))]
+CASES += [(abi.SHAPE_GRANITE, s, T) for s, T in ((4000, 3), (2191, 5), (1367, 8), (1216, 9), (1100, 16), (1130, 31),
+                                                 (620, 33), (600, 63), (4033, 63), (64, 9), (700, 2))]
+
+
+@pytest.mark.parametrize("dt", [abi.F16, abi.BF16])
+@pytest.mark.parametrize("shape,start,T", CASES)
+def test_rows_match_float64(ctx, shape, dt, start, T):
+    q, k, v, out = rows(ctx, shape, dt, start, T, start + T)
+    worst = 0.0
+    for t in sorted({0, 1, T // 2, T - 2, T - 1}):
+        n = start + t + 1
+        worst = max(worst, rel_err(out[t], attend64(q[t], k[:n], v[:n], HEADS[shape][3])))
+    log(f"causal rows {shape} {dt} {start}+{T}: {worst:.2e}")
+    assert worst <= TOL_16
+
+
+@pytest.mark.parametrize("shape,dt", [(abi.SHAPE_QWEN3, abi.BF16), (abi.SHAPE_QWEN3, abi.F16),
+                                      (abi.SHAPE_GRANITE, abi.F16), (abi.SHAPE_GRANITE, abi.BF16)])
+@pytest.mark.parametrize("late", [1, 3, 4])
+def test_an_infinite_draft_value_stays_out_of_earlier_rows(ctx, shape, dt, late):
+    start, T, head, dim = 6000, 5, 1, 9
+    q, k, v, out = rows(ctx, shape, dt, start, T, late, plant=(late, head, dim))
+    hq, hk, d, scale = HEADS[shape]
+    group = hq // hk
+    for t in range(T):
+        n = start + t + 1
+        vals = np.where(np.isfinite(v[:n]), v[:n], 0.0)
+        ref = attend64(q[t], k[:n], vals, scale)
+        got = out[t].copy()
+        if t >= late:
+            # inf, or NaN where bf16's second piece of the probability is negative
+            assert not np.any(np.isfinite(got[head * group:(head + 1) * group, dim]))
+            got[head * group:(head + 1) * group, dim] = ref[head * group:(head + 1) * group, dim]
+        assert rel_err(got, ref) <= TOL_16, t
