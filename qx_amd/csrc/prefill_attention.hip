@@ -77,6 +77,18 @@ static bool prefill_on_decode(const ShapeDims& s, int key_dtype, int value_dtype
            rows_on_decode(s, key_dtype, value_dtype, start, tokens);
 }
 
+// Equal 16-bit caches take a query of another dtype on causal rows alone (the
+// pipelined kernel reads the cache's own), up to this many of them: a limit of
+// the call, so it does not follow rows_on_decode's crossover, which lies above
+// it everywhere.
+static bool takes_other_query(const ShapeDims& s, int key_dtype, uint32_t start, uint32_t tokens) {
+    if (tokens <= kDecodeRowsAlways) return true;
+    const uint64_t length = (uint64_t)start + tokens;
+    if (tokens >= 64) return false;
+    if (s.group >= 8) return (tokens - 6) * length <= 126000u;
+    return key_dtype == F16 ? start >= 64 && tokens * length <= 70000u : tokens * length <= 90000u;
+}
+
 // fp32 and mixed K/V caches at the Granite shape beyond a few rows take the
 // split-product kernel (prefill_f32.hip); Qwen-shape fp32 caches and
 // tiered values stay on causal decode rows.
@@ -120,6 +132,9 @@ hipError_t launch_prefill_attention(const ShapeDims& s, const KvLayer& kv, uint3
         return launch_prefill_f32(s, kv, start_position, tokens, query, query_dtype, out, out_dtype, workspace, st,
                                   dispatches);
     if (prefill_on_decode(s, kv.key_dtype, kv.value_dtype, start_position, tokens)) {
+        if (kv.key_dtype != F32 && kv.key_dtype == kv.value_dtype && kv.key_dtype != query_dtype &&
+            prefill_pipe_supported(s) && !takes_other_query(s, kv.key_dtype, start_position, tokens))
+            return hipErrorNotSupported;
         const DecodePlan p = plan_decode_causal(s, kv.key_dtype, kv.value_dtype, start_position, tokens);
         return launch_decode_causal_rows(s, kv, p, start_position, tokens, query, query_dtype, out, out_dtype, workspace,
                                          st, dispatches);

@@ -3,8 +3,8 @@ chunk of a prompt), where several rows share a workgroup
 (decode_mfma_rows_kernel): row counts around a workgroup's rows (two on the
 Qwen shape, eight on Granite's), contexts around the rules' lines and the
 split's granularity of 128, against float64 attention over the cache's rows at
-the 16-bit bar; and an infinite value in a later drafted row, which must not
-reach the rows before it."""
+the 16-bit bar; an infinite value in a later drafted row, which must not
+reach the rows before it; and the calls whose query dtype is refused."""
 import numpy as np
 import pytest
 import torch
@@ -75,3 +75,24 @@ def test_an_infinite_draft_value_stays_out_of_earlier_rows(ctx, shape, dt, late)
             assert not np.any(np.isfinite(got[head * group:(head + 1) * group, dim]))
             got[head * group:(head + 1) * group, dim] = ref[head * group:(head + 1) * group, dim]
         assert rel_err(got, ref) <= TOL_16, t
+
+
+@pytest.mark.parametrize("shape,dt,start,T,taken", [
+    (abi.SHAPE_QWEN3, abi.BF16, 12000, 16, True), (abi.SHAPE_QWEN3, abi.BF16, 13000, 16, False),
+    (abi.SHAPE_QWEN3, abi.F16, 15000, 8, True), (abi.SHAPE_GRANITE, abi.F16, 2000, 34, True),
+    (abi.SHAPE_GRANITE, abi.F16, 2100, 34, False), (abi.SHAPE_GRANITE, abi.BF16, 2600, 34, True),
+    (abi.SHAPE_GRANITE, abi.BF16, 2700, 34, False)])
+def test_a_query_of_another_dtype_is_taken_up_to_its_limit(ctx, shape, dt, start, T, taken):
+    """The limit is the call's own: (T - 6) x context of 126000 on the Qwen
+    shape, T x context of 70000 (f16) or 90000 (bf16) on Granite's."""
+    hq, hk, d, _ = HEADS[shape]
+    arena = rt.KvArena(ctx, shape, 1, 1, start + T, dt)
+    arena.set_len(start + T)
+    q = torch.zeros((T, hq, d), device="cuda")
+    with rt.Graph(ctx) as graph:
+        if taken:
+            rt.prefill_attention(graph, arena, 0, start, q)
+        else:
+            with pytest.raises(abi.QxhError) as e:
+                rt.prefill_attention(graph, arena, 0, start, q)
+            assert e.value.code == abi.QXH_ERR_UNSUPPORTED
