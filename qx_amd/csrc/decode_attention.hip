@@ -1007,16 +1007,20 @@ __global__ __launch_bounds__(64 * WAVES) void decode_mfma_kernel(DecodeArgs a) {
 // Causal rows of one sequence on the matrix cores (equal 16-bit caches): the
 // few-row prefill calls, a drafted block to verify.  A row attends all cached
 // positions but the last few, so a workgroup takes 16 / G rows at once,
-// their G heads each as the 16 columns of S^T, and streams its range of the
-// K/V rows once for all of them (decode_mfma_kernel, one row a workgroup,
+// their G heads each as the 16 columns of S^T (CB such column blocks over the
+// same tiles, rows_blocks), and streams its range of the K/V rows once for all of them (decode_mfma_kernel, one row a workgroup,
 // streams it once per row and leaves 16 - G columns idle).  Tiles, operands and
 // the two register sets are decode_mfma_body's; column (row t, head g) masks
 // positions past causal_start + t.  The partials are decode_combine_kernel's.
-// Bound by the K/V rows' round trips and the merge: 8 Qwen rows over 30000
-// positions (61 MB a layer) 29.4 us, 44.6 with a row a workgroup; 8 Granite
-// rows over 3900 8.2 against 10.6.
+// Bound by the rate at which a CU pulls K/V from the caches behind it, and by
+// the merge: with one block, 15 tiles a wave take 26 us and 5 take 13, the same
+// with twice the waves a CU and with the workgroups that share a range on one
+// XCD.  16 Qwen rows over 30000 positions (61 MB a layer) 47.9 us with one
+// block, 38.9 with two; 8 rows 44.6 with a row a workgroup, 32.2 with one
+// block, 29.5 with two; 8 Granite rows over 3900 10.6 with a row a workgroup,
+// 8.4 with one block.  A wave's sums reuse its V tile's LDS.
 // ---------------------------------------------------------------------------
-template <int D, int G, int KDT>
+template <int D, int G, int KDT, int CB>
 __global__ __launch_bounds__(256) void decode_mfma_rows_kernel(DecodeArgs a) {
     using M = MfmaT<KDT>;
     using vec = typename M::vec;
@@ -1024,10 +1028,11 @@ __global__ __launch_bounds__(256) void decode_mfma_rows_kernel(DecodeArgs a) {
     constexpr int KSTEPS = D / 32, DTILES = D / 16;
     constexpr int VROWB = D * 2 + 32;
     constexpr int VCH = 32 * D * 2 / 16 / 64;
-    constexpr uint32_t ROWS = 16 / G;
-    __shared__ __attribute__((aligned(16))) char vtile[WAVES][32 * VROWB];
-    __shared__ float sm_m[WAVES][16], sm_l[WAVES][16];
-    __shared__ __attribute__((aligned(16))) float sm_acc[WAVES][16][D];
+    constexpr uint32_t BROWS = 16 / G, ROWS = CB * BROWS;  // rows a column block, a workgroup
+    // a wave's V tile, and its columns' sums once its tiles are done
+    constexpr int WBYTES = 32 * VROWB > CB * 16 * D * 4 ? 32 * VROWB : CB * 16 * D * 4;
+    __shared__ __attribute__((aligned(16))) char vtile[WAVES][WBYTES];
+    __shared__ float sm_m[WAVES][CB * 16], sm_l[WAVES][CB * 16];
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int lg = lane >> 4, li = lane & 15;
@@ -1041,27 +1046,36 @@ __global__ __launch_bounds__(256) void decode_mfma_rows_kernel(DecodeArgs a) {
     const uint32_t common = a.causal_start + t0 + 1;  // positions every row of the workgroup attends
     const uint16_t* vhead = reinterpret_cast<const uint16_t*>(a.values) + (size_t)kvh * a.head_stride;
 
-    // column li: row t0 + li / G, head li % G
-    const uint32_t limit = min(r1, common + li / G);  // positions the column attends
-    vec qop[KSTEPS];
-    float mrun = kNegBig, lrun = 0.f;
-    f32x4 oacc[DTILES];
+    // column li of block b: row t0 + b * BROWS + li / G, head li % G
+    uint32_t limit[CB];  // positions the column attends
+    vec qop[CB][KSTEPS];
+    float mrun[CB], lrun[CB];
+    f32x4 oacc[CB][DTILES];
 #pragma unroll
-    for (int dt = 0; dt < DTILES; ++dt) oacc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < CB; ++b) {
+        limit[b] = min(r1, common + b * BROWS + li / G);
+        mrun[b] = kNegBig;
+        lrun[b] = 0.f;
+#pragma unroll
+        for (int dt = 0; dt < DTILES; ++dt) oacc[b][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     auto load_q = [&]() __attribute__((always_inline)) {
-        const uint32_t row = min(t0 + li / G, T - 1);  // past the call: computed, never stored
-        const size_t q0 = (((size_t)row * hkv + kvh) * G + li % G) * D;
-        if (a.query_dtype == KDT) {
 #pragma unroll
-            for (int ks = 0; ks < KSTEPS; ++ks)
-                qop[ks] = __builtin_bit_cast(vec, load16<false>(reinterpret_cast<const char*>(a.query) +
-                                                                (q0 + 32 * ks + 8 * lg) * 2));
-        } else {
+        for (int b = 0; b < CB; ++b) {
+            const uint32_t row = min(t0 + b * BROWS + li / G, T - 1);  // past the call: computed, never stored
+            const size_t q0 = (((size_t)row * hkv + kvh) * G + li % G) * D;
+            if (a.query_dtype == KDT) {
 #pragma unroll
-            for (int ks = 0; ks < KSTEPS; ++ks)
+                for (int ks = 0; ks < KSTEPS; ++ks)
+                    qop[b][ks] = __builtin_bit_cast(vec, load16<false>(reinterpret_cast<const char*>(a.query) +
+                                                                       (q0 + 32 * ks + 8 * lg) * 2));
+            } else {
 #pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    qop[ks][j] = M::cvt(load_any(a.query, q0 + 32 * ks + 8 * lg + j, a.query_dtype));
+                for (int ks = 0; ks < KSTEPS; ++ks)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        qop[b][ks][j] = M::cvt(load_any(a.query, q0 + 32 * ks + 8 * lg + j, a.query_dtype));
+            }
         }
     };
     auto compute = [&](uint32_t base, const u32x4 (&kr)[2][KSTEPS], const u32x4 (&vr)[VCH])
@@ -1088,66 +1102,76 @@ __global__ __launch_bounds__(256) void decode_mfma_rows_kernel(DecodeArgs a) {
             *reinterpret_cast<u32x4*>(vl + chunk / (D / 8) * VROWB + chunk % (D / 8) * 16) =
                 out ? u32x4{0u, 0u, 0u, 0u} : vr[cc];
         }
-        f32x4 sacc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+        vec phi[CB], plo[CB];
 #pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks)
+        for (int b = 0; b < CB; ++b) {
+            f32x4 sacc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-            for (int mt = 0; mt < 2; ++mt) sacc[mt] = M::mma(__builtin_bit_cast(vec, kr[mt][ks]), qop[ks], sacc[mt]);
-        float sv[8];
-        float tmax = -INFINITY;
+            for (int ks = 0; ks < KSTEPS; ++ks)
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
+                for (int mt = 0; mt < 2; ++mt)
+                    sacc[mt] = M::mma(__builtin_bit_cast(vec, kr[mt][ks]), qop[b][ks], sacc[mt]);
+            float sv[8];
+            float tmax = -INFINITY;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t pos = base + 16 * mt + 4 * lg + j;
-                const float v = pos < limit ? sacc[mt][j] * c : -INFINITY;
-                sv[mt * 4 + j] = v;
-                tmax = fmaxf(tmax, v);
+            for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t pos = base + 16 * mt + 4 * lg + j;
+                    const float v = pos < limit[b] ? sacc[mt][j] * c : -INFINITY;
+                    sv[mt * 4 + j] = v;
+                    tmax = fmaxf(tmax, v);
+                }
+            tmax = max_xor32(max_xor16(tmax));
+            const float mnew = fmaxf(mrun[b], tmax);
+            const float alpha = fast_exp2(mrun[b] - mnew);
+            mrun[b] = mnew;
+            float psum = 0.f;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const float p = fast_exp2(sv[k] - mnew);
+                psum += p;
+                const auto h = M::cvt(p);
+                phi[b][k] = h;
+                if constexpr (KDT == BF16) plo[b][k] = M::cvt(p - (float)h);
             }
-        tmax = max_xor32(max_xor16(tmax));
-        const float mnew = fmaxf(mrun, tmax);
-        const float alpha = fast_exp2(mrun - mnew);
-        mrun = mnew;
-        vec phi, plo;
-        float psum = 0.f;
+            lrun[b] = __builtin_fmaf(lrun[b], alpha, psum);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const float p = fast_exp2(sv[k] - mnew);
-            psum += p;
-            const auto h = M::cvt(p);
-            phi[k] = h;
-            if constexpr (KDT == BF16) plo[k] = M::cvt(p - (float)h);
+            for (int dt = 0; dt < DTILES; ++dt) oacc[b][dt] *= alpha;
         }
-        lrun = __builtin_fmaf(lrun, alpha, psum);
-#pragma unroll
-        for (int dt = 0; dt < DTILES; ++dt) oacc[dt] *= alpha;
         if (apart) {
             // the rows past `common` one by one, straight from the cache: lane
             // (g, i) adds to its own dims of column i where the column attends
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                float p = (float)phi[k];
-                if constexpr (KDT == BF16) p += (float)plo[k];
+            for (int b = 0; b < CB; ++b)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    float p = (float)phi[b][k];
+                    if constexpr (KDT == BF16) p += (float)plo[b][k];
 #pragma unroll 1
-                for (int g = 0; g < 4; ++g) {
-                    const uint32_t pos = base + 16 * (k >> 2) + 4 * g + (k & 3);
-                    const float pg = __shfl(p, 16 * g + li);
-                    if (pos < common || pos >= limit) continue;
+                    for (int g = 0; g < 4; ++g) {
+                        const uint32_t pos = base + 16 * (k >> 2) + 4 * g + (k & 3);
+                        const float pg = __shfl(p, 16 * g + li);
+                        if (pos < common || pos >= limit[b]) continue;
 #pragma unroll
-                    for (int dt = 0; dt < DTILES; ++dt)
+                        for (int dt = 0; dt < DTILES; ++dt)
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const uint16_t v = vhead[(size_t)pos * D + 16 * dt + 4 * lg + j];
-                            oacc[dt][j] = __builtin_fmaf(pg, KDT == F16 ? half_bits_to_f32(v) : bf16_to_f32(v), oacc[dt][j]);
-                        }
+                            for (int j = 0; j < 4; ++j) {
+                                const uint16_t v = vhead[(size_t)pos * D + 16 * dt + 4 * lg + j];
+                                oacc[b][dt][j] = __builtin_fmaf(
+                                    pg, KDT == F16 ? half_bits_to_f32(v) : bf16_to_f32(v), oacc[b][dt][j]);
+                            }
+                    }
                 }
-            }
         }
 #pragma unroll
         for (int dt = 0; dt < DTILES; ++dt) {
             const vec vop = __builtin_bit_cast(vec, vt_operand_rows32<VROWB>(vl, 0, 16 * dt, lg, li));
-            oacc[dt] = M::mma(vop, phi, oacc[dt]);
-            if constexpr (KDT == BF16) oacc[dt] = M::mma(vop, plo, oacc[dt]);
+#pragma unroll
+            for (int b = 0; b < CB; ++b) {
+                oacc[b][dt] = M::mma(vop, phi[b], oacc[b][dt]);
+                if constexpr (KDT == BF16) oacc[b][dt] = M::mma(vop, plo[b], oacc[b][dt]);
+            }
         }
     };
 
@@ -1186,16 +1210,20 @@ __global__ __launch_bounds__(256) void decode_mfma_rows_kernel(DecodeArgs a) {
     }
 
     // merge the waves: a thread owns four dims of a column at a time
-    lrun = sum_xor32(sum_xor16(lrun));
 #pragma unroll
-    for (int dt = 0; dt < DTILES; ++dt) *reinterpret_cast<f32x4*>(&sm_acc[wave][li][16 * dt + 4 * lg]) = oacc[dt];
-    if (lg == 0) {
-        sm_m[wave][li] = mrun;
-        sm_l[wave][li] = lrun;
+    for (int b = 0; b < CB; ++b) {
+        lrun[b] = sum_xor32(sum_xor16(lrun[b]));
+#pragma unroll
+        for (int dt = 0; dt < DTILES; ++dt)
+            *reinterpret_cast<f32x4*>(vl + ((16 * b + li) * D + 16 * dt + 4 * lg) * 4) = oacc[b][dt];
+        if (lg == 0) {
+            sm_m[wave][16 * b + li] = mrun[b];
+            sm_l[wave][16 * b + li] = lrun[b];
+        }
     }
     __syncthreads();
 #pragma unroll
-    for (int i = threadIdx.x; i < 16 * D / 4; i += 64 * WAVES) {
+    for (int i = threadIdx.x; i < CB * 16 * D / 4; i += 64 * WAVES) {
         const int col = i / (D / 4), d = 4 * (i % (D / 4));
         const uint32_t row = t0 + col / G, g = col % G;
         if (row >= T) continue;
@@ -1208,7 +1236,7 @@ __global__ __launch_bounds__(256) void decode_mfma_rows_kernel(DecodeArgs a) {
         for (int w = 0; w < WAVES; ++w) {
             const float f = fast_exp2(sm_m[w][col] - Mx);
             L = __builtin_fmaf(sm_l[w][col], f, L);
-            const f32x4 v = *reinterpret_cast<const f32x4*>(&sm_acc[w][col][d]);
+            const f32x4 v = *reinterpret_cast<const f32x4*>(vtile[w] + (col * D + d) * 4);
 #pragma unroll
             for (int j = 0; j < 4; ++j) A[j] = __builtin_fmaf(v[j], f, A[j]);
         }
@@ -1737,17 +1765,46 @@ static bool rows_on_mfma(const ShapeDims& s, int key_dtype, int value_dtype, uin
     return pairs >= 11000 && length > (tokens >= 16 && tokens <= 32 ? 1152u : 640u);
 }
 
+// Column blocks of 16 a workgroup takes.  Two halve the K/V each CU pulls from
+// the caches behind it, which bounds long Qwen contexts, but split the range
+// over half as many workgroups' rows and leave up to three of the last four
+// rows empty.  Measured, us per call (one block / two, Qwen bf16): 8000 + 3
+// 12.9 / 14.5, 4000 + 16 15.1 / 16.4, 12000 + 5 18.5 / 18.9, 8000 + 16 20.3 /
+// 20.2, 30000 + 4 23.9 / 22.3, 24000 + 8 27.2 / 24.5, 30000 + 16 47.9 / 38.9,
+// 16000 + 24 44.5 / 37.4; with two or three rows empty 12000 + 9 20.8 / 22.3,
+// 20000 + 5 22.5 / 23.5, 30000 + 5 28.2 / 28.6.  Granite, with 8 rows a block
+// and a quarter of the bytes, only lost: 800 + 48 8.7 / 9.7, 3900 + 24 9.8 /
+// 10.4.
+static int rows_blocks(const ShapeDims& s, uint32_t tokens, uint32_t length) {
+    if (s.group < 8 || tokens < 3) return 1;
+    const bool full = tokens % 4 == 0 || tokens % 4 == 3;
+    return (uint64_t)tokens * length >= (full ? 100000u : 200000u) ? 2 : 1;
+}
+
+// One workgroup a CU, of at least a tile a wave: 192 and 384 workgroups, and
+// splits of 256 positions, measured the same or slower (Qwen 12000 + 8, one
+// column block, 192 / 256 / 384 workgroups 20.0 / 17.8 / 24.0 us).
+constexpr uint32_t kRowsGran = kWaves * 32;
+static uint32_t rows_splits(const ShapeDims& s, uint32_t tokens, uint32_t length) {
+    const uint32_t per = 16 / (uint32_t)s.group * rows_blocks(s, tokens, length);
+    const uint32_t units = (uint32_t)s.kv_heads * ((tokens + per - 1) / per);
+    return std::max(1u, std::min(kDecodeCus / units, (length + kRowsGran - 1) / kRowsGran));
+}
+
+// The most splits a call of `tokens` rows takes at any start: they grow with
+// the length, and rounding the chunk up only lowers them.
+static uint32_t rows_most_splits(const ShapeDims& s, int key_dtype, int value_dtype, uint32_t tokens,
+                                 uint32_t capacity) {
+    if (key_dtype != value_dtype || (key_dtype != F16 && key_dtype != BF16)) return 1;
+    return rows_splits(s, tokens, capacity);
+}
+
 static DecodePlan plan_rows_mfma(const ShapeDims& s, uint32_t start, uint32_t tokens) {
     DecodePlan p{};
     p.waves = kWaves;
-    const uint32_t per = 16 / (uint32_t)s.group, length = start + tokens;
-    const uint32_t units = (uint32_t)s.kv_heads * ((tokens + per - 1) / per);
-    // one workgroup a CU, of at least a tile a wave: 192 and 384 workgroups,
-    // and splits of 256 positions, measured the same or slower (Qwen 12000 +
-    // 8, 192 / 256 / 384 workgroups 20.0 / 17.8 / 24.0 us)
-    const uint32_t gran = kWaves * 32;
-    const uint32_t splits = std::max(1u, std::min(kDecodeCus / units, (length + gran - 1) / gran));
-    p.chunk = ((length + splits - 1) / splits + gran - 1) / gran * gran;
+    const uint32_t length = start + tokens;
+    const uint32_t splits = rows_splits(s, tokens, length);
+    p.chunk = ((length + splits - 1) / splits + kRowsGran - 1) / kRowsGran * kRowsGran;
     p.splits = (length + p.chunk - 1) / p.chunk;
     p.workspace_bytes =
         p.splits > 1 ? (uint64_t)tokens * s.kv_heads * p.splits * s.group * (s.head_dim + 2) * sizeof(float) : 0;
@@ -1760,13 +1817,17 @@ static hipError_t launch_rows_mfma(const ShapeDims& s, const KvLayer& kv, const 
         a.ws_ml = reinterpret_cast<float*>(workspace);
         a.ws_acc = a.ws_ml + 2 * (uint64_t)tokens * s.kv_heads * p.splits * s.group;
     }
-    const uint32_t per = 16 / (uint32_t)s.group;
-    const dim3 grid(p.splits, s.kv_heads, (tokens + per - 1) / per), block(64 * kWaves);
+    const int blocks = rows_blocks(s, tokens, a.length);
+    const uint32_t per = 16 / (uint32_t)s.group * blocks;
+    const dim3 grid(p.splits, s.kv_heads, (tokens + per - 1) / per);
     const bool granite = s.head_dim == 64 && s.group == 2, f16 = kv.key_dtype == F16;
-    if (granite && f16) hipLaunchKernelGGL((decode_mfma_rows_kernel<64, 2, F16>), grid, block, 0, st, a);
-    else if (granite) hipLaunchKernelGGL((decode_mfma_rows_kernel<64, 2, BF16>), grid, block, 0, st, a);
-    else if (f16) hipLaunchKernelGGL((decode_mfma_rows_kernel<128, 8, F16>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((decode_mfma_rows_kernel<128, 8, BF16>), grid, block, 0, st, a);
+    const dim3 block(64 * kWaves);
+    if (granite && f16) hipLaunchKernelGGL((decode_mfma_rows_kernel<64, 2, F16, 1>), grid, block, 0, st, a);
+    else if (granite) hipLaunchKernelGGL((decode_mfma_rows_kernel<64, 2, BF16, 1>), grid, block, 0, st, a);
+    else if (f16 && blocks == 1) hipLaunchKernelGGL((decode_mfma_rows_kernel<128, 8, F16, 1>), grid, block, 0, st, a);
+    else if (blocks == 1) hipLaunchKernelGGL((decode_mfma_rows_kernel<128, 8, BF16, 1>), grid, block, 0, st, a);
+    else if (f16) hipLaunchKernelGGL((decode_mfma_rows_kernel<128, 8, F16, 2>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((decode_mfma_rows_kernel<128, 8, BF16, 2>), grid, block, 0, st, a);
     *dispatches = 1;
     if (p.splits > 1) {
         const dim3 cgrid(s.q_heads * (s.head_dim / kCombineDims), tokens);
@@ -1801,6 +1862,8 @@ uint64_t decode_causal_workspace_bound(const ShapeDims& s, int key_dtype, int va
     uint32_t bound = want < cap ? want : cap;
     if (bound > (uint32_t)kMaxSplits) bound = kMaxSplits;
     if (bound < p.splits) bound = p.splits;
+    const uint32_t most = rows_most_splits(s, key_dtype, value_dtype, tokens, capacity);
+    if (bound < most) bound = most;
     return bound > 1 ? (uint64_t)units * bound * s.group * (s.head_dim + 2) * sizeof(float) : 0;
 }
 

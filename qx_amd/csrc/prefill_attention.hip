@@ -42,9 +42,10 @@ constexpr uint32_t kExactPassWgs = 256;
 // take otherwise (rows / tiled, us, 9-63 rows over 64-30000 cached positions,
 // each case timed both ways in one process; several rows share a workgroup,
 // decode_mfma_rows_kernel):
-// - Qwen (450000 up to 32 rows, 300000 beyond): 30000 + 12 39.5 / 64.1, 30000
-//   + 24 69.8 / 64.3, 16000 + 24 43.6 / 49.1, 16000 + 32 49.7 / 49.3, 8000 +
-//   32 31.0 / 43.9, 4000 + 63 33.7 / 37.8, 8000 + 48 50.4 / 43.6;
+// - Qwen (960000 up to 32 rows, 500000 beyond): 30000 + 16 38.9 / 66.1, 16000
+//   + 32 41.2 / 50.1, 24000 + 32 54.4 / 59.6, 30000 + 24 54.0 / 66.2, 30000 +
+//   32 64.4 / 66.3, 8000 + 48 38.2 / 44.0, 12000 + 48 47.4 / 48.2, 8000 + 63
+//   44.8 / 44.2, 16000 + 63 70.4 / 51.2;
 // - Granite f16 (500000, and at least 64 cached positions) and bf16 (500000):
 //   the rows win over the whole range, f16 250 + 9 3.9 / 8.7, 2000 + 48 9.9 /
 //   14.6, 3900 + 63 12.6 / 19.5, bf16 3900 + 63 13.2 / 22.3;
@@ -65,7 +66,7 @@ static bool rows_on_decode(const ShapeDims& s, int key_dtype, int value_dtype, u
     if (tokens >= 64) return false;
     const uint64_t length = (uint64_t)start + tokens;
     if (s.group >= 8)
-        return tokens * length <= (value_dtype == I8T ? 150000u : tokens <= 32 ? 450000u : 300000u);
+        return tokens * length <= (value_dtype == I8T ? 150000u : tokens <= 32 ? 960000u : 500000u);
     if (prefill_f32_supported(s, key_dtype, value_dtype)) return tokens * length <= 22000u;
     if (key_dtype == F16 && value_dtype == F16) return start >= 64 && tokens * length <= 500000u;
     if (key_dtype == BF16 && value_dtype == BF16) return tokens * length <= 500000u;

@@ -1,7 +1,7 @@
 """Few causal rows over equal 16-bit caches (a drafted block to verify, a short
 chunk of a prompt), where several rows share a workgroup
-(decode_mfma_rows_kernel): row counts around a workgroup's rows (two on the
-Qwen shape, eight on Granite's), contexts around the rules' lines and the
+(decode_mfma_rows_kernel): row counts around a workgroup's rows (two or four on
+the Qwen shape, eight on Granite's), contexts around the rules' lines and the
 split's granularity of 128, against float64 attention over the cache's rows at
 the 16-bit bar; an infinite value in a later drafted row, which must not
 reach the rows before it; and the calls whose query dtype is refused."""
@@ -40,7 +40,10 @@ def rows(ctx, shape, dt, start, T, seed, plant=None):
 
 
 CASES = [(abi.SHAPE_QWEN3, s, T) for s, T in ((9999, 2), (6700, 3), (4091, 5), (2490, 8), (2220, 9), (1250, 17),
-                                              (640, 32), (2528, 33), (2500, 63), (100, 63), (3000, 2))]
+                                              (640, 32), (2528, 33), (2500, 63), (100, 63), (3000, 2),
+                                              # two column blocks a workgroup: full and ragged last fours
+                                              (33400, 3), (25100, 4), (40000, 5), (14280, 7), (7000, 15),
+                                              (6100, 33), (29900, 32), (1530, 63), (7870, 63))]
 CASES += [(abi.SHAPE_GRANITE, s, T) for s, T in ((4000, 3), (2191, 5), (1367, 8), (1216, 9), (1100, 16), (1130, 31),
                                                  (620, 33), (600, 63), (4033, 63), (64, 9), (700, 2))]
 
@@ -59,9 +62,10 @@ def test_rows_match_float64(ctx, shape, dt, start, T):
 
 @pytest.mark.parametrize("shape,dt", [(abi.SHAPE_QWEN3, abi.BF16), (abi.SHAPE_QWEN3, abi.F16),
                                       (abi.SHAPE_GRANITE, abi.F16), (abi.SHAPE_GRANITE, abi.BF16)])
-@pytest.mark.parametrize("late", [1, 3, 4])
-def test_an_infinite_draft_value_stays_out_of_earlier_rows(ctx, shape, dt, late):
-    start, T, head, dim = 6000, 5, 1, 9
+@pytest.mark.parametrize("start,T,late", [(6000, 5, 1), (6000, 5, 3), (6000, 5, 4),
+                                          (14300, 7, 1), (14300, 7, 2), (14300, 7, 5)])
+def test_an_infinite_draft_value_stays_out_of_earlier_rows(ctx, shape, dt, start, T, late):
+    head, dim = 1, 9
     q, k, v, out = rows(ctx, shape, dt, start, T, late, plant=(late, head, dim))
     hq, hk, d, scale = HEADS[shape]
     group = hq // hk
