@@ -642,7 +642,7 @@ def bench_prefill_fp32(ctx, steps, warmup):
         torch.cuda.empty_cache()
     res["note"] = ("Granite causal prefill of 2048 tokens, fp32 queries and outputs; fp32k_tiered: fp32 K with "
                    "tiered values (f16 window of 256 rows, block INT8 below); peak = dense fp32 MFMA "
-                   "(157.3 TFLOP/s); flop = 4*D*Hq*T(T+1)/2")
+                   "(157.3 TFLOP/s), which 16-bit piece products can pass; flop = 4*D*Hq*T(T+1)/2")
     return res
 
 
