@@ -40,9 +40,9 @@
 // read with 16-byte loads, split once per workgroup and written to LDS as one
 // 8 KB plane per piece, 16-byte chunks XOR-swizzled by row & 7 (conflict-free
 // for both kinds of operand read); the next tile's loads are in flight while
-// the current one is computed.  Scores are scaled by softmax scale x log2(e)
-// in fp32 after the dot product and exponentiated with v_exp_f32; the online
-// softmax keeps per-column (m, l) in every lane.
+// the current one is computed.  The online softmax keeps per-column (m, l) in
+// every lane, m a score as the product left it; a score's distance from it is
+// scaled by softmax scale x log2(e) in fp32 and exponentiated with v_exp_f32.
 //
 // A piece of an infinity, or a product that overflows where the whole one
 // does not, would turn into a NaN, so a workgroup that meets a magnitude of
@@ -61,7 +61,7 @@ namespace qxh {
 namespace {
 
 constexpr int kD = 64;
-constexpr float kNegBigF = -1.0e30f;
+constexpr float kNoScore = -3.4028234e38f;   // the running maximum before any score
 constexpr int kTierBlockF32 = 32;           // elements per INT8 scale block of a tiered value cache
 constexpr int kPlaneBytes = kPrefillTile * kD * 2;
 constexpr float kSplitLimit = 0x1p60f;      // magnitudes the split products take
@@ -258,6 +258,7 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
     constexpr int NK = KIo::PIECES, NV = VIo::PIECES;
     constexpr bool kHalfV = VDT == F16;
     constexpr float kShift = kHalfV ? 12.0f : 0.0f;  // exponent offset of the probabilities
+    constexpr float kUnshift = kHalfV ? 0x1p-12f : 1.0f;
     constexpr int kStageBytes = (NK + NV) * kPlaneBytes;
     // two stages where two workgroups of them still share a CU's 160 KB
     constexpr int STAGES = kStageBytes < 40 * 1024 ? 2 : 1;
@@ -366,7 +367,10 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
     for (int db = 0; db < 4; ++db)
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) oacc[db][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float mrun[2] = {kNegBigF, kNegBigF}, lsum[2] = {0.f, 0.f};
+    // The running maximum is a score as the product left it: the exponent of
+    // its own probability is then exactly zero at any magnitude (scaled first,
+    // the rounding of a large score would be left in the exponent).
+    float smrun[2] = {kNoScore, kNoScore}, lsum[2] = {0.f, 0.f};
 
     // operand addresses inside a stage: K rows 16 pb + i, chunk 4 h + g; V
     // rows 32 h + 4 g + i / 4 (+ 16), dims 16 db + 4 (i % 4)
@@ -438,16 +442,15 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
 #pragma unroll
                 for (int j = 0; j < 4; ++j) smax = fmaxf(smax, sacc[pb][nt][j]);
             smax = max_xor32(max_xor16(smax));
-            const float mnew = fmaxf(mrun[nt], smax * c);
-            const float alpha = fast_exp2(mrun[nt] - mnew);
-            mrun[nt] = mnew;
-            const float off = kShift - mnew;
+            const float mnew = fmaxf(smrun[nt], smax);
+            const float alpha = fast_exp2((smrun[nt] - mnew) * c);
+            smrun[nt] = mnew;
             float ps = 0.0f;
 #pragma unroll
             for (int pb = 0; pb < 4; ++pb)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const float p = fast_exp2(__builtin_fmaf(sacc[pb][nt][j], c, off));
+                    const float p = fast_exp2(__builtin_fmaf(sacc[pb][nt][j] - mnew, c, kShift));
                     sacc[pb][nt][j] = p;
                     ps += p;
                 }
@@ -556,12 +559,12 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
         for (int nt = 0; nt < 2; ++nt) {
             const size_t colx = slot + wave * 32 + nt * 16 + li;
             if (lg == 0) {
-                a.part_ml[2 * colx] = mrun[nt] - kShift;  // l and O carry the offset
-                a.part_ml[2 * colx + 1] = lsum[nt];
+                a.part_ml[2 * colx] = smrun[nt] * c;
+                a.part_ml[2 * colx + 1] = lsum[nt] * kUnshift;
             }
 #pragma unroll
             for (int db = 0; db < 4; ++db)
-                *reinterpret_cast<f32x4*>(a.part_o + colx * kD + 16 * db + 4 * lg) = oacc[db][nt];
+                *reinterpret_cast<f32x4*>(a.part_o + colx * kD + 16 * db + 4 * lg) = oacc[db][nt] * kUnshift;
         }
         return;
     }

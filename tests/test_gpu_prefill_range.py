@@ -1,0 +1,100 @@
+"""The range of the fp32 and mixed-cache prefill (prefill_f32.hip): scores of any
+size, infinities and NaN in later rows of the call, a large value under a small
+weight, values next to either end of binary32, and the bits of each product.
+Reference: float64 attention over the cache's own rows, within the fp32 bar's
+5e-6 of the row's RMS unless a test derives its own."""
+import numpy as np
+import pytest
+import torch
+
+from qx_amd import abi
+from qx_amd import runtime as rt
+from tests.helpers import TOL_F32, attend64, log, rel_err
+
+pytestmark = pytest.mark.gpu
+
+SCALE = 0.015625
+PLANS = [(abi.F32, abi.F16), (abi.F32, abi.F32), (abi.F32, abi.BF16), (abi.F16, abi.F32), (abi.BF16, abi.F32),
+         (abi.F32, abi.I8_TIERED)]
+WIDE_KEYS = [(k, v) for k, v in PLANS if k != abi.F16]  # keys past binary16's range
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    return rt.Context(0)
+
+
+def prefill(ctx, k, v, q, kdt, vdt, start):
+    """k, v: [start + T][8][64] fp32; q: [T][16][64]; returns out and the cache's rows."""
+    cap = k.shape[0]
+    window = 64 if vdt == abi.I8_TIERED else 0
+    arena = rt.KvArena(ctx, abi.SHAPE_GRANITE, 1, 1, cap, kdt, vdt, value_window=window)
+    with rt.Graph(ctx) as g:
+        rt.store_kv(g, arena, 0, 0, k[None].cuda(), v[None].cuda())
+        out = rt.prefill_attention(g, arena, 0, start, q.cuda())
+        kk, vv = arena.gather(g, 0, 0, 0, cap)
+    return out.cpu().numpy(), kk.float().cpu().numpy(), vv.float().cpu().numpy()
+
+
+def inputs(n, T, seed):
+    g = torch.Generator().manual_seed(seed)
+    k, v = (torch.randn((n, 8, 64), generator=g) for _ in range(2))
+    return k, v, torch.randn((T, 16, 64), generator=g)
+
+
+def check(out, q, kk, vv, start, rows, tol=TOL_F32 / 2):
+    worst = 0.0
+    for t in rows:
+        n = start + t + 1
+        e = rel_err(out[t], attend64(q[t].numpy(), kk[:n], vv[:n], SCALE))
+        assert e <= tol, (t, e)
+        worst = max(worst, e)
+    return worst
+
+
+# ---- large scores -----------------------------------------------------------------
+
+@pytest.mark.parametrize("kdt,vdt", PLANS)
+@pytest.mark.parametrize("size", [1e4, 3e4])
+def test_large_scores(ctx, kdt, vdt, size):
+    """Scores up to 2^29 in the exponent's units, too far apart for a second
+    position to count: the largest of a row weighs exactly one, and the row is
+    that position's values."""
+    start, T = 70, 100
+    k, v, q = inputs(start + T, T, int(size))
+    k, q = (size * k).clamp(-65504, 65504), size * q
+    out, kk, vv = prefill(ctx, k, v, q, kdt, vdt, start)
+    check(out, q, kk, vv, start, [0, 1, 57, 58, T - 1])
+
+
+@pytest.mark.parametrize("kdt,vdt", WIDE_KEYS)
+@pytest.mark.parametrize("power", [40, 59, 60, 64, 90])
+def test_large_keys_under_ordinary_queries(ctx, kdt, vdt, power):
+    """One dim decides every score, alike in no two positions (nor in bf16)."""
+    T = 150
+    k, v, q = inputs(T, T, power)
+    k[:, :, 5] = torch.sign(k[:, :, 5]) * (1 + torch.arange(T)[:, None]) * 2.0 ** power
+    out, kk, vv = prefill(ctx, k, v, q, kdt, vdt, 0)
+    check(out, q, kk, vv, 0, [0, 63, 64, 100, T - 1])
+
+
+@pytest.mark.parametrize("kdt,vdt", PLANS)
+@pytest.mark.parametrize("power", [59, 64, 90])
+def test_large_queries_over_ordinary_keys(ctx, kdt, vdt, power):
+    T = 150
+    k, v, q = inputs(T, T, power + 1)
+    q[::3, :, 5] *= 2.0 ** power
+    out, kk, vv = prefill(ctx, k, v, q, kdt, vdt, 0)
+    check(out, q, kk, vv, 0, [0, 1, 63, 64, 99, T - 1])
+
+
+@pytest.mark.parametrize("kdt,vdt", PLANS)
+def test_a_query_past_the_limit_with_keys_as_small(ctx, kdt, vdt):
+    """Queries of 2^64 over keys of 2^-64 (2^-14 in binary16, where the query's
+    is 2^14): ordinary scores on the path of large magnitudes."""
+    T, power = 150, 14 if kdt == abi.F16 else 64
+    k, v, q = inputs(T, T, 64)
+    k[:, :, 5] *= 2.0 ** -power
+    q[:, :, 5] *= 2.0 ** power
+    out, kk, vv = prefill(ctx, k, v, q, kdt, vdt, 0)
+    check(out, q, kk, vv, 0, [0, 63, 64, 100, T - 1])
