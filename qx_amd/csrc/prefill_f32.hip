@@ -46,8 +46,9 @@
 //
 // A piece of an infinity, or a product that overflows where the whole one
 // does not, would turn into a NaN, so a workgroup that meets a magnitude of
-// 2^60 or more (a non-finite f16 value, say) takes that tile's two products
-// on the fp32 matrix cores, straight from the cache.
+// 2^60 or more (a non-finite f16 value, say) or a NaN takes that tile's two
+// products on the fp32 matrix cores, straight from the cache, and keeps what a
+// column does not attend out of its sums.
 #include <algorithm>
 #include <type_traits>
 
@@ -112,11 +113,14 @@ __device__ __forceinline__ uint32_t round_f16(float a, float b, uint32_t& rest) 
     return w;
 }
 
+// NaN if one of them is (v_maximum3_f32, two values an instruction).
 __device__ __forceinline__ float max_abs8(const float (&f)[8], float m) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) m = fmaxf(m, __builtin_fabsf(f[i]));
+    for (int i = 0; i < 8; ++i) m = __builtin_elementwise_maximum(m, __builtin_fabsf(f[i]));
     return m;
 }
+
+__device__ __forceinline__ bool finite(float x) { return (__float_as_uint(x) & 0x7f800000u) != 0x7f800000u; }
 
 // Byte offset of 16-byte chunk `col` of tile row `row` in a plane.
 __device__ __forceinline__ int plane_chunk(int row, int col) { return row * (kD * 2) + ((col ^ (row & 7)) << 4); }
@@ -141,7 +145,7 @@ template <int DT, bool VALUES> struct SplitIo {
             for (int i = 0; i < WORDS; ++i) raw.w[k][i] = load16<false>(p + 16 * i);
         }
     }
-    // returns whether a magnitude reaches the split's limit
+    // returns whether a magnitude reaches the split's limit or is NaN
     __device__ __forceinline__ static bool store(const Raw& raw, char* lds, int tid) {
         float m = 0.0f;
 #pragma unroll
@@ -170,7 +174,7 @@ template <int DT, bool VALUES> struct SplitIo {
                 for (int i = 0; i < PIECES; ++i) *reinterpret_cast<u32x4*>(dst + i * kPlaneBytes) = p[i];
             }
         }
-        return m >= (DT == F16 ? 65536.0f : kSplitLimit);
+        return !(m < (DT == F16 ? 65536.0f : kSplitLimit));
     }
     __device__ __forceinline__ static float at(const PrefillPipeArgs&, const char* base, uint32_t, uint32_t row,
                                                int dim) {
@@ -230,7 +234,7 @@ struct TieredSplitIo {
             for (int i = 0; i < 3; ++i)
                 *reinterpret_cast<u32x4*>(lds + i * kPlaneBytes + plane_chunk(tid >> 2, 2 * (tid & 3) + k)) = p[i];
         }
-        return m >= kSplitLimit;
+        return !(m < kSplitLimit);
     }
     __device__ __forceinline__ static float at(const PrefillPipeArgs& a, const char*, uint32_t kvh, uint32_t row,
                                                int dim) {
@@ -357,7 +361,7 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
             mq = max_abs8(f, mq);
             split8<3>(f, q[x >> 1][x & 1]);
         }
-        qwide = mq >= kSplitLimit;
+        qwide = !(mq < kSplitLimit);
     }
     store_tile(t0, 0);
     __syncthreads();
@@ -460,19 +464,56 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
         }
         // O^T += V^T . P^T
         if (!split) {
+            // A masked position has weight zero, and zero times an infinity is
+            // NaN: past the positions that every column of the wave attends,
+            // the matrix product takes finite values only, and the others go
+            // one by one to the columns that attend them.
+            const uint32_t common = a.start + w_t0 + 1;
+            uint32_t apart = 0;  // bit 4 pb + j: this lane's value at that position is one of them
 #pragma unroll
             for (int pb = 0; pb < 4; ++pb)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const uint32_t row = min(kt * kPrefillTile + 16 * pb + 4 * (uint32_t)(l >> 4) + j, kv_len - 1);
+                    const uint32_t pos = kt * kPrefillTile + 16 * pb + 4 * (uint32_t)(l >> 4) + j;
 #pragma unroll
                     for (int db = 0; db < 4; ++db) {
-                        const float v = VIo::at(a, vbase, kvh, row, 16 * db + (l & 15));
+                        float v = VIo::at(a, vbase, kvh, min(pos, kv_len - 1), 16 * db + (l & 15));
+                        if (pos >= common && !finite(v)) {
+                            v = 0.0f;
+                            apart |= 1u << (4 * pb + j);
+                        }
 #pragma unroll
                         for (int nt = 0; nt < 2; ++nt) oacc[db][nt] = mma4(v, sacc[pb][nt][j], oacc[db][nt]);
                     }
                     __builtin_amdgcn_sched_barrier(0);  // few registers before many loads in flight
                 }
+            const uint32_t end = min((kt + 1) * kPrefillTile, a.start + w_last + 1);
+#pragma unroll 1
+            for (uint32_t pos = max(common, kt * kPrefillTile); pos < end; ++pos) {
+                const uint32_t bit = (pos >> 2 & 12) | (pos & 3);
+                const int group = pos >> 2 & 3;  // of lanes that holds the position
+                if (!__any((l >> 4) == group && (apart >> bit & 1))) continue;
+                float p[2] = {0.0f, 0.0f};
+#pragma unroll
+                for (int b = 0; b < 16; ++b)
+                    if (bit == (uint32_t)b) {
+                        p[0] = sacc[b >> 2][0][b & 3];
+                        p[1] = sacc[b >> 2][1][b & 3];
+                    }
+#pragma unroll
+                for (int nt = 0; nt < 2; ++nt) p[nt] = __shfl(p[nt], 16 * group + (l & 15));
+                if (pos > qpos) continue;
+#pragma unroll
+                for (int db = 0; db < 4; ++db)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const float v = VIo::at(a, vbase, kvh, pos, 16 * db + 4 * (l >> 4) + j);
+                        if (finite(v)) continue;
+#pragma unroll
+                        for (int nt = 0; nt < 2; ++nt)
+                            oacc[db][nt][j] = __builtin_fmaf(p[nt], v, oacc[db][nt][j]);
+                    }
+            }
             return;
         }
         const char* vt = st + NK * kPlaneBytes;

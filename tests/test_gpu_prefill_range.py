@@ -98,3 +98,45 @@ def test_a_query_past_the_limit_with_keys_as_small(ctx, kdt, vdt):
     q[:, :, 5] *= 2.0 ** power
     out, kk, vv = prefill(ctx, k, v, q, kdt, vdt, 0)
     check(out, q, kk, vv, 0, [0, 63, 64, 100, T - 1])
+
+
+# ---- infinities and NaN in later rows of the call ---------------------------------------
+
+@pytest.mark.parametrize("kdt,vdt,bad", [(k, v, b) for k, v in PLANS if v != abi.I8_TIERED
+                                         for b in (float("inf"), float("-inf"), float("nan"))] +
+                         [(abi.F32, abi.F16, 1e5)])
+@pytest.mark.parametrize("start,T,late", [(2400, 16, 15), (1600, 24, 7), (750, 48, 31), (0, 130, 70), (1400, 16, 12)])
+def test_a_later_rows_value_stays_out_of_earlier_rows(ctx, kdt, vdt, bad, start, T, late):
+    """A value that is no number, or that overflows the cache's binary16, in one
+    row of the call: the rows before it do not see it, the rows from it on are
+    not finite in its dim alone."""
+    k, v, q = inputs(start + T, T, start + T)
+    head, dim = 3, 11
+    v[start + late, head, dim] = bad
+    out, kk, vv = prefill(ctx, k, v, q, kdt, vdt, start)
+    finite = np.where(np.isfinite(vv), vv, 0.0)
+    check(out, q, kk, finite, start, [0, late // 2, late - 1])
+    assert not np.any(np.isfinite(out[late:, 2 * head:2 * head + 2, dim]))
+    out[late:, 2 * head:2 * head + 2, dim] = 0.0
+    for t in (late, T - 1):
+        ref = attend64(q[t].numpy(), kk[:start + t + 1], finite[:start + t + 1], SCALE)
+        ref[2 * head:2 * head + 2, dim] = 0.0
+        assert rel_err(out[t], ref) <= TOL_F32 / 2, t
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_a_later_rows_value_in_the_tiered_window(ctx, bad):
+    start, T, late = 3050, 16, 12
+    k, v, q = inputs(start + T, T, 5)
+    v[start + late, 3, 11] = bad
+    out, kk, vv = prefill(ctx, k, v, q, abi.F32, abi.I8_TIERED, start)
+    check(out, q, kk, np.where(np.isfinite(vv), vv, 0.0), start, [0, late - 1])
+
+
+@pytest.mark.parametrize("vdt", [abi.F16, abi.F32, abi.BF16])
+def test_a_later_rows_key_stays_out_of_earlier_rows(ctx, vdt):
+    start, T, late = 2400, 16, 12
+    k, v, q = inputs(start + T, T, 6)
+    k[start + late, 3, 11] = float("nan")
+    out, kk, vv = prefill(ctx, k, v, q, abi.F32, vdt, start)
+    check(out, q, np.where(np.isfinite(kk), kk, 0.0), vv, start, [0, late - 1])
