@@ -8,22 +8,22 @@
 //
 //   x = x0 + x1 + x2      bf16: x0 the top 8 bits, x1 and x2 the remainders
 //                         rounded to nearest; f16 values are two pieces and
-//                         bf16 values one, exactly
+//                         bf16 values one, exactly.  bf16 has fp32's exponents,
+//                         so a small probability keeps its bits as well (as f16
+//                         pieces, below 2^-15 of the largest, it lost them: 4e-4
+//                         of the result where a large value has a weight of
+//                         2^-24)
 //   x . y = sum of xi . yj with i + j <= 2 (what is left out is below 2^-24
 //                         of the product), accumulated in fp32, the small
 //                         products first
 //
-// Probabilities over f16 values (exact as they are) are two f16 pieces, held
-// to 2^-23; their exponent is offset by 2^12 so that the second piece stays
-// clear of f16's subnormals.  Against 64 bits the result is as close as the
-// fp32 matrix cores' was or closer (1900 tokens: 2.6e-7 of the result against
-// 3.3e-7 on Fp32KFp16V; 3000 tokens of fp32 K/V: 3.5e-7 against 4.6e-7).
+// Against 64 bits the result is as close as the fp32 matrix cores' was or
+// closer.
 //
-// Bound: at 1900 tokens of Fp32KFp16V 128 MFMAs a tile and wave (2048 cycles
-// of matrix core; 8192 on the fp32 cores) run in about 45 us, against 88 on
-// the fp32 cores; the matrix core is busy a quarter of that, the rest is the
-// softmax and the split of the tile on the VALU, waits, and the start of each
-// workgroup (query pieces, first tile).
+// Bound: a tile of Fp32KFp16V is 176 MFMAs a wave (2816 cycles of matrix core;
+// 8192 on the fp32 cores), beside the softmax and the split of the tile and of
+// the probabilities on the VALU.  1900 tokens take 70 us a layer, 97 on the
+// fp32 cores.
 //
 // Transposed FlashAttention-2 on 16x16x32 MFMAs (operand layout: mfma.h):
 //
@@ -71,7 +71,6 @@ __device__ __forceinline__ f32x4 mma4(float a, float b, const f32x4& c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 // bf16 pieces of the pair (a, b), packed (a in the low half).  x0 is cut off,
@@ -100,19 +99,6 @@ template <int NP> __device__ __forceinline__ void split8(float (&f)[8], u32x4 (&
     }
 }
 
-// f16 pieces of the pair (a, b): the pair rounded to nearest, and what that
-// left of it (exact before its own rounding; one v_fma_mix per value).
-__device__ __forceinline__ uint32_t round_f16(float a, float b, uint32_t& rest) {
-    const uint32_t w = __builtin_bit_cast(uint32_t, f16x2{(_Float16)a, (_Float16)b});
-    uint32_t r;
-    asm("v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]\n\t"
-        "v_fma_mixhi_f16 %0, %1, -1.0, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
-        : "=&v"(r)
-        : "v"(w), "v"(a), "v"(b));
-    rest = r;
-    return w;
-}
-
 // NaN if one of them is (v_maximum3_f32, two values an instruction).
 __device__ __forceinline__ float max_abs8(const float (&f)[8], float m) {
 #pragma unroll
@@ -126,11 +112,10 @@ __device__ __forceinline__ bool finite(float x) { return (__float_as_uint(x) & 0
 __device__ __forceinline__ int plane_chunk(int row, int col) { return row * (kD * 2) + ((col ^ (row & 7)) << 4); }
 
 // A 64 x 64 tile of one dtype: thread t moves chunks of 8 elements, chunk k at
-// row t / 8 + 32 k, elements 8 (t % 8) .. + 7.  PIECES planes; as values an
-// f16 tile stays f16 (VALUES), as keys it is two bf16 pieces.
-template <int DT, bool VALUES> struct SplitIo {
+// row t / 8 + 32 k, elements 8 (t % 8) .. + 7, and writes PIECES planes.
+template <int DT> struct SplitIo {
     static constexpr int EB = DT == F32 ? 4 : 2;
-    static constexpr int PIECES = DT == F32 ? 3 : DT == F16 && !VALUES ? 2 : 1;
+    static constexpr int PIECES = DT == F32 ? 3 : DT == F16 ? 2 : 1;
     static constexpr int WORDS = DT == F32 ? 2 : 1;  // 16-byte loads a chunk
     struct Raw {
         u32x4 w[2][WORDS];
@@ -257,12 +242,9 @@ __device__ __forceinline__ f32x4 mma_bf(const u32x4& a, const u32x4& b, const f3
 // grid (qblocks x kv_heads, chunks of the longest block), block 256.
 template <int KDT, int VDT>
 __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) {
-    using KIo = SplitIo<KDT, false>;
-    using VIo = std::conditional_t<VDT == I8T, TieredSplitIo, SplitIo<VDT == I8T ? F16 : VDT, true>>;
+    using KIo = SplitIo<KDT>;
+    using VIo = std::conditional_t<VDT == I8T, TieredSplitIo, SplitIo<VDT == I8T ? F16 : VDT>>;
     constexpr int NK = KIo::PIECES, NV = VIo::PIECES;
-    constexpr bool kHalfV = VDT == F16;
-    constexpr float kShift = kHalfV ? 12.0f : 0.0f;  // exponent offset of the probabilities
-    constexpr float kUnshift = kHalfV ? 0x1p-12f : 1.0f;
     constexpr int kStageBytes = (NK + NV) * kPlaneBytes;
     // two stages where two workgroups of them still share a CU's 160 KB
     constexpr int STAGES = kStageBytes < 40 * 1024 ? 2 : 1;
@@ -454,7 +436,7 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
             for (int pb = 0; pb < 4; ++pb)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const float p = fast_exp2(__builtin_fmaf(sacc[pb][nt][j] - mnew, c, kShift));
+                    const float p = fast_exp2((sacc[pb][nt][j] - mnew) * c);
                     sacc[pb][nt][j] = p;
                     ps += p;
                 }
@@ -527,51 +509,26 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
         };
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            if constexpr (kHalfV) {
-                f16x8 p0[2], p1[2];
+            u32x4 p[2][3];
 #pragma unroll
-                for (int nt = 0; nt < 2; ++nt) {
-                    u32x4 w, rest;
+            for (int nt = 0; nt < 2; ++nt) {
+                float f[8];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const f32x4& s = sacc[2 * h + (e >> 1)][nt];
-                        uint32_t x;
-                        w[e] = round_f16(s[2 * (e & 1)], s[2 * (e & 1) + 1], x);
-                        rest[e] = x;
-                    }
-                    p0[nt] = __builtin_bit_cast(f16x8, w);
-                    p1[nt] = __builtin_bit_cast(f16x8, rest);
-                }
+                for (int e = 0; e < 8; ++e) f[e] = sacc[2 * h + (e >> 2)][nt][e & 3];
+                split8<3>(f, p[nt]);
+            }
 #pragma unroll
-                for (int db = 0; db < 4; ++db) {
-                    const f16x8 v = __builtin_bit_cast(f16x8, v_operand(h, 0, db));
+            for (int db = 0; db < 4; ++db) {
+                u32x4 v[NV];
 #pragma unroll
-                    for (int nt = 0; nt < 2; ++nt) oacc[db][nt] = MfmaT<F16>::mma(v, p1[nt], oacc[db][nt]);
+                for (int i = 0; i < NV; ++i) v[i] = __builtin_bit_cast(u32x4, v_operand(h, i, db));
 #pragma unroll
-                    for (int nt = 0; nt < 2; ++nt) oacc[db][nt] = MfmaT<F16>::mma(v, p0[nt], oacc[db][nt]);
-                }
-            } else {
-                u32x4 p[2][3];
+                for (int sum = 2; sum >= 0; --sum)
 #pragma unroll
-                for (int nt = 0; nt < 2; ++nt) {
-                    float f[8];
+                    for (int i = 0; i < NV; ++i)
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) f[e] = sacc[2 * h + (e >> 2)][nt][e & 3];
-                    split8<3>(f, p[nt]);
-                }
-#pragma unroll
-                for (int db = 0; db < 4; ++db) {
-                    u32x4 v[NV];
-#pragma unroll
-                    for (int i = 0; i < NV; ++i) v[i] = __builtin_bit_cast(u32x4, v_operand(h, i, db));
-#pragma unroll
-                    for (int sum = 2; sum >= 0; --sum)
-#pragma unroll
-                        for (int i = 0; i < NV; ++i)
-#pragma unroll
-                            for (int nt = 0; nt < 2; ++nt)
-                                if (i <= sum) oacc[db][nt] = mma_bf(v[i], p[nt][sum - i], oacc[db][nt]);
-                }
+                        for (int nt = 0; nt < 2; ++nt)
+                            if (i <= sum) oacc[db][nt] = mma_bf(v[i], p[nt][sum - i], oacc[db][nt]);
             }
         }
     };
@@ -601,11 +558,11 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
             const size_t colx = slot + wave * 32 + nt * 16 + li;
             if (lg == 0) {
                 a.part_ml[2 * colx] = smrun[nt] * c;
-                a.part_ml[2 * colx + 1] = lsum[nt] * kUnshift;
+                a.part_ml[2 * colx + 1] = lsum[nt];
             }
 #pragma unroll
             for (int db = 0; db < 4; ++db)
-                *reinterpret_cast<f32x4*>(a.part_o + colx * kD + 16 * db + 4 * lg) = oacc[db][nt] * kUnshift;
+                *reinterpret_cast<f32x4*>(a.part_o + colx * kD + 16 * db + 4 * lg) = oacc[db][nt];
         }
         return;
     }

@@ -140,3 +140,25 @@ def test_a_later_rows_key_stays_out_of_earlier_rows(ctx, vdt):
     k[start + late, 3, 11] = float("nan")
     out, kk, vv = prefill(ctx, k, v, q, abi.F32, vdt, start)
     check(out, q, np.where(np.isfinite(kk), kk, 0.0), vv, start, [0, late - 1])
+
+
+# ---- weights and values of all sizes ------------------------------------------------------
+
+@pytest.mark.parametrize("kdt,vdt", PLANS)
+@pytest.mark.parametrize("bits", [12, 16, 20, 24, 27, 30])
+def test_a_large_value_under_a_small_weight(ctx, kdt, vdt, bits):
+    """One position of weight 2^-bits whose value outweighs all the others': its
+    weight counts with all of its bits.  (Tiered values hold it in the binary16
+    window.)"""
+    start, T = 60, 64
+    n = start + T
+    k, v, q = inputs(n, T, bits)
+    k.zero_()
+    q.fill_(1.0)
+    at = start + 1  # in the window of the last 64 positions, seen by every row but the first
+    k[at] = -round((bits + 0.3) * np.log(2.0) * 4) / 4  # 64 dims of it times 1/64, exact in any sum
+    v *= 2.0 ** -18
+    v[at] = 60000.0 * (1 + torch.arange(64) / 100.0) / 2
+    out, kk, vv = prefill(ctx, k, v, q, kdt, vdt, start)
+    e = check(out, q, kk, vv, start, [1, 2, 3, 40, T - 1])
+    log(f"large value under 2^-{bits} {kdt}/{vdt}: vs float64 {e:.2e}")
