@@ -6,16 +6,18 @@
 // into 16-bit pieces that hold all of its 24 significand bits, and each
 // product is the sum of the piece products that matter:
 //
-//   x = x0 + x1 + x2      bf16: x0 the top 8 bits, x1 and x2 the remainders
-//                         rounded to nearest; f16 values are two pieces and
+//   x = x0 + x1 + x2      bf16: x0 is x rounded to nearest, x1 and x2 what is
+//                         left rounded to nearest; f16 values are two pieces and
 //                         bf16 values one, exactly.  bf16 has fp32's exponents,
 //                         so a small probability keeps its bits as well (as f16
 //                         pieces, below 2^-15 of the largest, it lost them: 4e-4
 //                         of the result where a large value has a weight of
 //                         2^-24)
-//   x . y = sum of xi . yj with i + j <= 2 (what is left out is below 2^-24
-//                         of the product), accumulated in fp32, the small
-//                         products first
+//   x . y = sum of xi . yj with i + j <= 2, accumulated in fp32, the small
+//                         products first.  |x1| <= 2^-8 and |x2| <= 2^-17 of x's
+//                         leading bit, so x1 y2 + x2 y1, which is left out, is at
+//                         most 2^-24 of the product, what an fp32 product is
+//                         rounded by (2^-22 where x0 was cut off instead)
 //
 // Against 64 bits the result is as close as the fp32 matrix cores' was or
 // closer.
@@ -73,15 +75,8 @@ __device__ __forceinline__ f32x4 mma4(float a, float b, const f32x4& c) {
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
-// bf16 pieces of the pair (a, b), packed (a in the low half).  x0 is cut off,
-// not rounded: the pieces of a finite value are finite.
-__device__ __forceinline__ uint32_t top_bf16(float& a, float& b) {
-    const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
-    const uint32_t w = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
-    a -= __uint_as_float(ua & 0xffff0000u);
-    b -= __uint_as_float(ub & 0xffff0000u);
-    return w;
-}
+// The next bf16 piece of the pair (a, b), packed (a in the low half), rounded
+// to nearest; what it leaves of them stays in a and b.
 __device__ __forceinline__ uint32_t round_bf16(float& a, float& b) {
     const uint32_t w = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)a, (__bf16)b});
     a -= __uint_as_float(w << 16);
@@ -92,11 +87,9 @@ __device__ __forceinline__ uint32_t round_bf16(float& a, float& b) {
 // 8 values as NP packed bf16 pieces (the values are used up).
 template <int NP> __device__ __forceinline__ void split8(float (&f)[8], u32x4 (&p)[NP]) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        p[0][i] = top_bf16(f[2 * i], f[2 * i + 1]);
-        if constexpr (NP > 1) p[1][i] = round_bf16(f[2 * i], f[2 * i + 1]);
-        if constexpr (NP > 2) p[2][i] = round_bf16(f[2 * i], f[2 * i + 1]);
-    }
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int n = 0; n < NP; ++n) p[n][i] = round_bf16(f[2 * i], f[2 * i + 1]);
 }
 
 // NaN if one of them is (v_maximum3_f32, two values an instruction).

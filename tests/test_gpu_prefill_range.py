@@ -162,3 +162,29 @@ def test_a_large_value_under_a_small_weight(ctx, kdt, vdt, bits):
     out, kk, vv = prefill(ctx, k, v, q, kdt, vdt, start)
     e = check(out, q, kk, vv, start, [1, 2, 3, 40, T - 1])
     log(f"large value under 2^-{bits} {kdt}/{vdt}: vs float64 {e:.2e}")
+
+
+# ---- the bits of a product -------------------------------------------------------------
+
+@pytest.mark.parametrize("vdt", [abi.F16, abi.F32])
+@pytest.mark.parametrize("bits", [0x3f80ff80, 0x3f807f80, 0x3f817fc0])
+def test_product_bits(ctx, vdt, bits):
+    """Two keys of nearly one score, one of the query's own 17 bits a dim and one
+    of 8: the first needs every product of pieces.  Their values are 1 and -1,
+    so the result errs by half of the scores' error.  In units of 2^-24 of the
+    score: at most 1 is left out by the pieces and 1 goes to the rounding of
+    each sum; a leading piece that is cut off leaves out up to 4."""
+    x = np.array([bits], np.uint32).view(np.float32)[0].item()
+    near = float(torch.tensor(x).to(torch.bfloat16))
+    T, big = 64, 32.0
+    k = torch.full((T, 8, 64), -big)  # the other positions weigh nothing
+    v = torch.zeros((T, 8, 64))
+    q = torch.full((T, 16, 64), x * big)
+    k[0], k[1] = x * big, near * big
+    v[0], v[1] = 1.0, -1.0
+    out, kk, vv = prefill(ctx, k, v, q, abi.F32, vdt, 0)
+    ref = attend64(q[1].numpy(), kk[:2], vv[:2], SCALE)
+    unit = big * big * x * x * 64 * SCALE * 2.0 ** -24
+    err = np.max(np.abs(out[1:] - ref)) * 2 / unit
+    log(f"score error {err:.2f} units of 2^-24")
+    assert err <= 3
