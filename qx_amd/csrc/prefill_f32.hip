@@ -47,10 +47,14 @@
 // scaled by softmax scale x log2(e) in fp32 and exponentiated with v_exp_f32.
 //
 // A piece of an infinity, or a product that overflows where the whole one
-// does not, would turn into a NaN, so a workgroup that meets a magnitude of
-// 2^60 or more (a non-finite f16 value, say) or a NaN takes that tile's two
-// products on the fp32 matrix cores, straight from the cache, and keeps what a
-// column does not attend out of its sums.
+// does not, would turn into a NaN, and the last piece of a value near fp32's
+// least would lose bits below bf16's least, so a workgroup that meets a
+// magnitude of 2^60 or more (a non-finite f16 value, say), a NaN, or an fp32
+// value below 2^-80 that is not zero takes that tile's two products on the fp32
+// matrix cores, straight from the cache, and keeps what a column does not
+// attend out of its sums.  Keys and queries need no such least: what a piece
+// loses there is below 2^-60 of a score's unit.  Nor do probabilities: a piece
+// loses less than 2^-126 of the largest one, and v_exp_f32 itself ends there.
 #include <algorithm>
 #include <type_traits>
 
@@ -68,6 +72,7 @@ constexpr float kNoScore = -3.4028234e38f;   // the running maximum before any s
 constexpr int kTierBlockF32 = 32;           // elements per INT8 scale block of a tiered value cache
 constexpr int kPlaneBytes = kPrefillTile * kD * 2;
 constexpr float kSplitLimit = 0x1p60f;      // magnitudes the split products take
+constexpr float kSplitLeast = 0x1p-80f;     // and the least of a value that is not zero
 
 __device__ __forceinline__ f32x4 mma4(float a, float b, const f32x4& c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -99,6 +104,14 @@ __device__ __forceinline__ float max_abs8(const float (&f)[8], float m) {
     return m;
 }
 
+// The least magnitude that is not zero (and m), as 2 |x| - 1 in its bits: zero
+// wraps around to the largest.
+__device__ __forceinline__ uint32_t min_bits8(const float (&f)[8], uint32_t m) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m = min(m, (__float_as_uint(f[i]) << 1) - 1u);
+    return m;
+}
+
 __device__ __forceinline__ bool finite(float x) { return (__float_as_uint(x) & 0x7f800000u) != 0x7f800000u; }
 
 // Byte offset of 16-byte chunk `col` of tile row `row` in a plane.
@@ -106,7 +119,7 @@ __device__ __forceinline__ int plane_chunk(int row, int col) { return row * (kD 
 
 // A 64 x 64 tile of one dtype: thread t moves chunks of 8 elements, chunk k at
 // row t / 8 + 32 k, elements 8 (t % 8) .. + 7, and writes PIECES planes.
-template <int DT> struct SplitIo {
+template <int DT, bool VALUES> struct SplitIo {
     static constexpr int EB = DT == F32 ? 4 : 2;
     static constexpr int PIECES = DT == F32 ? 3 : DT == F16 ? 2 : 1;
     static constexpr int WORDS = DT == F32 ? 2 : 1;  // 16-byte loads a chunk
@@ -123,9 +136,11 @@ template <int DT> struct SplitIo {
             for (int i = 0; i < WORDS; ++i) raw.w[k][i] = load16<false>(p + 16 * i);
         }
     }
-    // returns whether a magnitude reaches the split's limit or is NaN
+    // returns whether a magnitude is outside of the split's range or NaN
     __device__ __forceinline__ static bool store(const Raw& raw, char* lds, int tid) {
+        constexpr bool kLeast = VALUES && DT == F32;
         float m = 0.0f;
+        uint32_t least = ~0u;
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
             char* dst = lds + plane_chunk((tid >> 3) + 32 * k, tid & 7);
@@ -143,6 +158,7 @@ template <int DT> struct SplitIo {
                 Unpack<DT>::run(raw.w[k][0], f);
             }
             m = max_abs8(f, m);
+            if constexpr (kLeast) least = min_bits8(f, least);
             if constexpr (PIECES == 1) {
                 *reinterpret_cast<u32x4*>(dst) = raw.w[k][0];
             } else {
@@ -152,7 +168,8 @@ template <int DT> struct SplitIo {
                 for (int i = 0; i < PIECES; ++i) *reinterpret_cast<u32x4*>(dst + i * kPlaneBytes) = p[i];
             }
         }
-        return !(m < (DT == F16 ? 65536.0f : kSplitLimit));
+        return !(m < (DT == F16 ? 65536.0f : kSplitLimit)) ||
+               (kLeast && least < (__builtin_bit_cast(uint32_t, kSplitLeast) << 1) - 1u);
     }
     __device__ __forceinline__ static float at(const PrefillPipeArgs&, const char* base, uint32_t, uint32_t row,
                                                int dim) {
@@ -235,8 +252,8 @@ __device__ __forceinline__ f32x4 mma_bf(const u32x4& a, const u32x4& b, const f3
 // grid (qblocks x kv_heads, chunks of the longest block), block 256.
 template <int KDT, int VDT>
 __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) {
-    using KIo = SplitIo<KDT>;
-    using VIo = std::conditional_t<VDT == I8T, TieredSplitIo, SplitIo<VDT == I8T ? F16 : VDT>>;
+    using KIo = SplitIo<KDT, false>;
+    using VIo = std::conditional_t<VDT == I8T, TieredSplitIo, SplitIo<VDT == I8T ? F16 : VDT, true>>;
     constexpr int NK = KIo::PIECES, NV = VIo::PIECES;
     constexpr int kStageBytes = (NK + NV) * kPlaneBytes;
     // two stages where two workgroups of them still share a CU's 160 KB

@@ -164,6 +164,32 @@ def test_a_large_value_under_a_small_weight(ctx, kdt, vdt, bits):
     log(f"large value under 2^-{bits} {kdt}/{vdt}: vs float64 {e:.2e}")
 
 
+@pytest.mark.parametrize("kdt,vdt", [(k, v) for k, v in PLANS if v in (abi.F32, abi.BF16)])
+@pytest.mark.parametrize("power", [-118, -112, -105, -60, 50, 59, 61, 100, 118])
+def test_values_near_the_ends_of_binary32(ctx, kdt, vdt, power):
+    """Values of one far magnitude, under weights within 2^-2 of each other."""
+    T = 200
+    k, v, q = inputs(T, T, power + 200)
+    v *= 2.0 ** power
+    out, kk, vv = prefill(ctx, k, v, q, kdt, vdt, 0)
+    for t in [0, 63, 64, 150, T - 1]:
+        ref = attend64(q[t].numpy(), kk[:t + 1], vv[:t + 1], SCALE)
+        e = rel_err(out[t] * 2.0 ** -power, ref * 2.0 ** -power)
+        assert e <= TOL_F32 / 2, (t, e)
+
+
+@pytest.mark.parametrize("kdt,vdt", [(k, v) for k, v in PLANS if v in (abi.F32, abi.BF16)])
+def test_small_and_large_tiles_in_one_call(ctx, kdt, vdt):
+    """Tiles of every range in turn, so that the sums pass from one way of
+    forming the products to the other and back; each weighed so as to count."""
+    T = 320
+    k, v, q = inputs(T, T, 3)
+    for tile, power in enumerate((0, 70, 3, -110, 66)):
+        v[64 * tile:64 * tile + 64] *= 2.0 ** power
+    out, kk, vv = prefill(ctx, k, v, q, kdt, vdt, 0)
+    check(out, q, kk, vv, 0, [0, 63, 64, 130, 200, 300, T - 1])
+
+
 # ---- the bits of a product -------------------------------------------------------------
 
 @pytest.mark.parametrize("vdt", [abi.F16, abi.F32])
