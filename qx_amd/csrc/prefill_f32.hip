@@ -117,6 +117,19 @@ __device__ __forceinline__ bool finite(float x) { return (__float_as_uint(x) & 0
 // Byte offset of 16-byte chunk `col` of tile row `row` in a plane.
 __device__ __forceinline__ int plane_chunk(int row, int col) { return row * (kD * 2) + ((col ^ (row & 7)) << 4); }
 
+// 16 consecutive elements of a row, widened (the fp32 path's operands).
+template <int DT> __device__ __forceinline__ void load_row16(const void* base, size_t idx, float (&f)[16]) {
+    const char* p = reinterpret_cast<const char*>(base) + idx * (DT == F32 ? 4 : 2);
+    constexpr int E = DT == F32 ? 4 : 8;  // elements a load
+#pragma unroll
+    for (int i = 0; i < 16 / E; ++i) {
+        float x[E];
+        Unpack<DT>::run(load16<false>(p + 16 * i), x);
+#pragma unroll
+        for (int e = 0; e < E; ++e) f[E * i + e] = x[e];
+    }
+}
+
 // A 64 x 64 tile of one dtype: thread t moves chunks of 8 elements, chunk k at
 // row t / 8 + 32 k, elements 8 (t % 8) .. + 7, and writes PIECES planes.
 template <int DT, bool VALUES> struct SplitIo {
@@ -402,21 +415,28 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
                 sacc[pb][1] = acc[1];
             }
         } else {
+            // contraction slot s of lane group g is dim 16 g + s in both operands
+            const size_t qr = ((size_t)min(w_t0 + (l & 15), T - 1) * a.q_heads + (size_t)kvh * 2) * kD + 16 * (l >> 4);
+            float qf[2][16];
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt) {
+                if (a.query_dtype == F32) load_row16<F32>(a.query, qr + nt * kD, qf[nt]);
+                else if (a.query_dtype == F16) load_row16<F16>(a.query, qr + nt * kD, qf[nt]);
+                else load_row16<BF16>(a.query, qr + nt * kD, qf[nt]);
+            }
 #pragma unroll
             for (int pb = 0; pb < 4; ++pb) {
                 const uint32_t row = min(kt * kPrefillTile + 16 * pb + (uint32_t)(l & 15), kv_len - 1);
-                const size_t qr = ((size_t)min(w_t0 + (l & 15), T - 1) * a.q_heads + (size_t)kvh * 2) * kD;
+                float k[16];
+                load_row16<KDT>(kbase, (size_t)row * kD + 16 * (l >> 4), k);
                 f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-#pragma unroll 1
-                for (int s = 0; s < 16; ++s) {
-                    const int dim = 32 * (s >> 3) + 8 * (l >> 4) + (s & 7);
-                    const float k = KIo::at(a, kbase, kvh, row, dim);
 #pragma unroll
-                    for (int nt = 0; nt < 2; ++nt)
-                        acc[nt] = mma4(k, load_any(a.query, qr + nt * kD + dim, a.query_dtype), acc[nt]);
-                }
+                for (int s = 0; s < 16; ++s)
+#pragma unroll
+                    for (int nt = 0; nt < 2; ++nt) acc[nt] = mma4(k[s], qf[nt][s], acc[nt]);
                 sacc[pb][0] = acc[0];
                 sacc[pb][1] = acc[1];
+                __builtin_amdgcn_sched_barrier(0);  // few registers before many loads in flight
             }
         }
         // causal mask, online softmax per column
@@ -463,22 +483,27 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
             const uint32_t common = a.start + w_t0 + 1;
             uint32_t apart = 0;  // bit 4 pb + j: this lane's value at that position is one of them
 #pragma unroll
-            for (int pb = 0; pb < 4; ++pb)
+            for (int pb = 0; pb < 4; ++pb) {
+                const uint32_t pos = kt * kPrefillTile + 16 * pb + 4 * (uint32_t)(l >> 4);
+                float v[4][4];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t pos = kt * kPrefillTile + 16 * pb + 4 * (uint32_t)(l >> 4) + j;
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int db = 0; db < 4; ++db)
+                        v[j][db] = VIo::at(a, vbase, kvh, min(pos + j, kv_len - 1), 16 * db + (l & 15));
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
 #pragma unroll
                     for (int db = 0; db < 4; ++db) {
-                        float v = VIo::at(a, vbase, kvh, min(pos, kv_len - 1), 16 * db + (l & 15));
-                        if (pos >= common && !finite(v)) {
-                            v = 0.0f;
+                        if (pos + j >= common && !finite(v[j][db])) {
+                            v[j][db] = 0.0f;
                             apart |= 1u << (4 * pb + j);
                         }
 #pragma unroll
-                        for (int nt = 0; nt < 2; ++nt) oacc[db][nt] = mma4(v, sacc[pb][nt][j], oacc[db][nt]);
+                        for (int nt = 0; nt < 2; ++nt) oacc[db][nt] = mma4(v[j][db], sacc[pb][nt][j], oacc[db][nt]);
                     }
-                    __builtin_amdgcn_sched_barrier(0);  // few registers before many loads in flight
-                }
+                __builtin_amdgcn_sched_barrier(0);  // few registers before many loads in flight
+            }
             const uint32_t end = min((kt + 1) * kPrefillTile, a.start + w_last + 1);
 #pragma unroll 1
             for (uint32_t pos = max(common, kt * kPrefillTile); pos < end; ++pos) {
