@@ -450,6 +450,7 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
                     for (int nt = 0; nt < 2; ++nt) sacc[pb][nt][j] = pos <= qpos ? sacc[pb][nt][j] : -INFINITY;
                 }
         }
+        float alpha[2];
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
             float smax = -INFINITY;
@@ -459,7 +460,7 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
                 for (int j = 0; j < 4; ++j) smax = fmaxf(smax, sacc[pb][nt][j]);
             smax = max_xor32(max_xor16(smax));
             const float mnew = fmaxf(smrun[nt], smax);
-            const float alpha = fast_exp2((smrun[nt] - mnew) * c);
+            alpha[nt] = fast_exp2((smrun[nt] - mnew) * c);
             smrun[nt] = mnew;
             float ps = 0.0f;
 #pragma unroll
@@ -470,9 +471,7 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
                     sacc[pb][nt][j] = p;
                     ps += p;
                 }
-            lsum[nt] = __builtin_fmaf(lsum[nt], alpha, ps);
-#pragma unroll
-            for (int db = 0; db < 4; ++db) oacc[db][nt] *= alpha;
+            lsum[nt] = __builtin_fmaf(lsum[nt], alpha[nt], ps);
         }
         // O^T += V^T . P^T
         if (!split) {
@@ -481,6 +480,10 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
             // the matrix product takes finite values only, and the others go
             // one by one to the columns that attend them.
             const uint32_t common = a.start + w_t0 + 1;
+#pragma unroll
+            for (int db = 0; db < 4; ++db)
+#pragma unroll
+                for (int nt = 0; nt < 2; ++nt) oacc[db][nt] *= alpha[nt];
             uint32_t apart = 0;  // bit 4 pb + j: this lane's value at that position is one of them
 #pragma unroll
             for (int pb = 0; pb < 4; ++pb) {
@@ -542,29 +545,40 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
             const i16x4 r1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(p + 16 * kD * 2));
             return __builtin_shufflevector(r0, r1, 0, 1, 2, 3, 4, 5, 6, 7);
         };
+        // the tile's products are summed by themselves and added to O once: the
+        // running sums of a long chain are rounded once a tile
+        u32x4 p[2][2][3];  // [h][head][piece]
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            u32x4 p[2][3];
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
             for (int nt = 0; nt < 2; ++nt) {
                 float f[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) f[e] = sacc[2 * h + (e >> 2)][nt][e & 3];
-                split8<3>(f, p[nt]);
+                split8<3>(f, p[h][nt]);
             }
 #pragma unroll
-            for (int db = 0; db < 4; ++db) {
-                u32x4 v[NV];
+        for (int db = 0; db < 4; ++db) {
+            f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+            u32x4 v[2][NV];
 #pragma unroll
-                for (int i = 0; i < NV; ++i) v[i] = __builtin_bit_cast(u32x4, v_operand(h, i, db));
+            for (int h = 0; h < 2; ++h)
 #pragma unroll
-                for (int sum = 2; sum >= 0; --sum)
+                for (int i = 0; i < NV; ++i) v[h][i] = __builtin_bit_cast(u32x4, v_operand(h, i, db));
 #pragma unroll
-                    for (int i = 0; i < NV; ++i)
+            for (int sum = 2; sum >= 0; --sum)
+#pragma unroll
+                for (int i = 0; i < NV; ++i)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
 #pragma unroll
                         for (int nt = 0; nt < 2; ++nt)
-                            if (i <= sum) oacc[db][nt] = mma_bf(v[i], p[nt][sum - i], oacc[db][nt]);
-            }
+                            if (i <= sum) acc[nt] = mma_bf(v[h][i], p[h][nt][sum - i], acc[nt]);
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    oacc[db][nt][j] = __builtin_fmaf(oacc[db][nt][j], alpha[nt], acc[nt][j]);
         }
     };
 
