@@ -669,9 +669,13 @@ static uint32_t f32_chunks(const ShapeDims& s, uint32_t tokens, uint32_t tiles) 
     return std::max(1u, std::min(kF32MaxChunks, std::max(fill, cut)));
 }
 
-// most chunks a block can take in a cache of `capacity` positions
+// Partial slots of a block in a cache of `capacity` positions: chunks for
+// kF32MostWgs workgroups, of a tile at least, which is no less than f32_chunks
+// takes at any start.  Over short caches it makes the size grow with the prompt,
+// so that a workspace asked for a program's longest prompt serves the others.
 static uint32_t f32_max_chunks(const ShapeDims& s, uint32_t tokens, uint32_t capacity) {
-    return f32_chunks(s, tokens, (capacity + kPrefillTile - 1) / kPrefillTile);
+    const uint32_t wgs = f32_blocks(s, tokens), tiles = (capacity + kPrefillTile - 1) / kPrefillTile;
+    return std::max(1u, std::min({kF32MaxChunks, (kF32MostWgs + wgs - 1) / wgs, tiles}));
 }
 
 static uint32_t f32_chunk_tiles(const ShapeDims& s, uint32_t start, uint32_t tokens) {

@@ -214,3 +214,22 @@ def test_product_bits(ctx, vdt, bits):
     err = np.max(np.abs(out[1:] - ref)) * 2 / unit
     log(f"score error {err:.2f} units of 2^-24")
     assert err <= 3
+
+
+# ---- workspace -------------------------------------------------------------------------
+
+@pytest.mark.parametrize("kdt,vdt", PLANS)
+@pytest.mark.parametrize("capacity", [300, 512, 1000])
+def test_a_workspace_of_a_long_prompt_serves_shorter_ones(ctx, kdt, vdt, capacity):
+    """A program asks once, for its longest prompt."""
+    window = 64 if vdt == abi.I8_TIERED else 0
+    arena = rt.KvArena(ctx, abi.SHAPE_GRANITE, 1, 1, capacity, kdt, vdt, value_window=window)
+    sizes = [rt.prefill_workspace_bytes(arena, t) for t in range(1, capacity + 1)]
+    assert sizes == sorted(sizes)
+    workspace = torch.empty(sizes[-1], dtype=torch.uint8, device="cuda")
+    q = torch.randn((127, 16, 64), device="cuda")
+    with rt.Graph(ctx) as g:
+        arena.fill_normal(g, seed=1, length=capacity)
+        want = rt.prefill_attention(g, arena, 0, capacity - 127, q)
+        out = rt.prefill_attention(g, arena, 0, capacity - 127, q, workspace=workspace)
+    assert torch.equal(out, want)
