@@ -628,22 +628,24 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillPipeArgs a) 
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-// Split KV.  A workgroup costs about 5 us beside its tiles (query pieces,
-// first tile, partials) and a tile about 3.2 us where two workgroups share a
-// CU, so a block's KV range is cut
+// Split KV.  The longest block's chain of tiles sets the time until the chip is
+// full, and each chunk costs a workgroup's start and a merge, so a block's KV
+// range is cut
 // - into enough chunks for kF32TargetWgs workgroups (two per CU), each at
-//   least kF32MinTiles tiles, and
+//   least kF32MinTiles tiles, or one where a block has kF32FewTiles at most, and
 // - into chunks of about kF32ChunkTiles tiles while that makes at most
 //   kF32MostWgs workgroups: with more blocks than CUs the longest block's
 //   chain would set the time.
-// Measured, Fp32KFp16V, us per layer of an 8-layer prompt (front end and
-// merge included), start + T: at least 8 tiles a chunk / this rule 0 + 256
-// 21.2 / 20.0, 0 + 512 30.9 / 23.3, 1000 + 100 35.5 / 22.8, 2000 + 500 47.5 /
-// 41.4; toward 512 workgroups only / this rule 0 + 3000 111.0 / 104.9; toward
-// 2048 with 2 tiles (the fp32 matrix cores' rule) / this rule 2000 + 500
-// 49.0 / 41.4, 0 + 3000 110.0 / 104.9, 0 + 1900 60.5 / 60.0.
+// Measured, Fp32KFp16V, us per layer of 8 (merge included), start + T: at least
+// 8 tiles a chunk / this rule 0 + 256 20.3 / 14.5, 0 + 700 43.8 / 25.4, 900 +
+// 100 35.9 / 19.6, 2000 + 500 58.3 / 45.8; two tiles at least throughout / this
+// rule 63 + 66 15.8 / 13.2, 100 + 64 17.1 / 13.3, 0 + 192 16.8 / 13.9; toward
+// 512 workgroups only / this rule 64 + 2999 138.0 / 126.7; toward 2048 with 2
+// tiles / this rule 2000 + 500 53.7 / 45.8, 1000 + 1000 65.3 / 58.1, 0 + 1900
+// 67.1 / 69.9.
 constexpr uint32_t kF32TargetWgs = 512;
 constexpr uint32_t kF32MinTiles = 2;
+constexpr uint32_t kF32FewTiles = 4;
 constexpr uint32_t kF32ChunkTiles = 8;
 constexpr uint32_t kF32MostWgs = 2048;
 constexpr uint32_t kF32MaxChunks = 32;
@@ -664,7 +666,7 @@ static uint32_t f32_blocks(const ShapeDims& s, uint32_t tokens) {
 // chunks of a block of `tiles` tiles
 static uint32_t f32_chunks(const ShapeDims& s, uint32_t tokens, uint32_t tiles) {
     const uint32_t wgs = f32_blocks(s, tokens);
-    const uint32_t fill = std::min((kF32TargetWgs + wgs - 1) / wgs, tiles / kF32MinTiles);
+    const uint32_t fill = std::min((kF32TargetWgs + wgs - 1) / wgs, tiles <= kF32FewTiles ? tiles : tiles / kF32MinTiles);
     const uint32_t cut = std::min(kF32MostWgs / wgs, tiles / kF32ChunkTiles);
     return std::max(1u, std::min(kF32MaxChunks, std::max(fill, cut)));
 }
