@@ -49,15 +49,14 @@ constexpr uint32_t kExactPassWgs = 256;
 // - Granite f16 (500000, and at least 64 cached positions) and bf16 (500000):
 //   the rows win over the whole range, f16 250 + 9 3.9 / 8.7, 2000 + 48 9.9 /
 //   14.6, 3900 + 63 12.6 / 19.5, bf16 3900 + 63 13.2 / 22.3;
-// - the Granite split-product kernel (fp32 and mixed caches; c = 0, 22000):
-//   Fp32KFp16V 1000 + 16 10.4 / 11.0, 500 + 32 12.1 / 12.9, 2000 + 9 13.6 /
-//   12.3, 1000 + 24 14.1 / 11.4, 500 + 48 14.4 / 13.2; fp32 K/V 500 + 48
-//   15.0 / 16.6, 1000 + 24 14.9 / 13.4; Fp16KFp32V 2000 + 9 13.2 / 13.7,
-//   1000 + 24 13.4 / 12.7 (70000 while it ran on the fp32 matrix cores:
-//   4000 + 16 22.2 / 15.6 went to the rows);
-// - the other Granite plans (tiered values): c = 0, 40000;
-// - Qwen with tiered values (c = 0, 150000), whose decode rows keep splits
-//   toward 2048 workgroups.
+// - the Granite split-product kernel (36000; fp32 keys with tiered values
+//   48500): Fp32KFp16V 500 + 63 16.9 / 19.4, 1000 + 32 18.2 / 19.0, 1500 + 24
+//   19.0 / 16.7; fp32 K/V 1000 + 32 19.9 / 20.9, 1500 + 24 20.5 / 18.1, 3000 +
+//   12 21.8 / 19.8; Fp16KFp32V 500 + 63 18.9 / 19.9, 4000 + 9 25.4 / 21.4;
+//   tiered 4000 + 9 20.7 / 24.2, 4000 + 12 20.4 / 24.4, 1500 + 32 19.9 / 18.4;
+// - the other Granite plans (tiered values with 16-bit keys): 40000;
+// - Qwen with tiered values (150000), whose decode rows keep splits toward
+//   2048 workgroups.
 // The former short-prompt kernel, one 8-head workgroup per kv head, took
 // 1.31 ms for 1-16 rows at 32764 Qwen positions.
 constexpr uint32_t kDecodeRowsAlways = 8;
@@ -67,7 +66,8 @@ static bool rows_on_decode(const ShapeDims& s, int key_dtype, int value_dtype, u
     const uint64_t length = (uint64_t)start + tokens;
     if (s.group >= 8)
         return tokens * length <= (value_dtype == I8T ? 150000u : tokens <= 32 ? 960000u : 500000u);
-    if (prefill_f32_supported(s, key_dtype, value_dtype)) return tokens * length <= 22000u;
+    if (prefill_f32_supported(s, key_dtype, value_dtype))
+        return tokens * length <= (value_dtype == I8T ? 48500u : 36000u);
     if (key_dtype == F16 && value_dtype == F16) return start >= 64 && tokens * length <= 500000u;
     if (key_dtype == BF16 && value_dtype == BF16) return tokens * length <= 500000u;
     return tokens * length <= 40000u;
