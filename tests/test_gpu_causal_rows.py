@@ -4,7 +4,8 @@ chunk of a prompt), where several rows share a workgroup
 the Qwen shape, eight on Granite's), contexts around the rules' lines and the
 split's granularity of 128, against float64 attention over the cache's rows at
 the 16-bit bar; an infinite value in a later drafted row, which must not
-reach the rows before it; and the calls whose query dtype is refused."""
+reach the rows before it; and queries of another dtype, rounded to the cache's
+or refused."""
 import numpy as np
 import pytest
 import torch
@@ -100,3 +101,28 @@ def test_a_query_of_another_dtype_is_taken_up_to_its_limit(ctx, shape, dt, start
             with pytest.raises(abi.QxhError) as e:
                 rt.prefill_attention(graph, arena, 0, start, q)
             assert e.value.code == abi.QXH_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("qdt", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape,dt,start,T", [
+    (abi.SHAPE_QWEN3, abi.BF16, 12000, 5), (abi.SHAPE_QWEN3, abi.F16, 12000, 13),  # one column block a workgroup
+    (abi.SHAPE_QWEN3, abi.BF16, 15000, 7), (abi.SHAPE_QWEN3, abi.F16, 15000, 8),  # two
+    (abi.SHAPE_QWEN3, abi.BF16, 10000, 12), (abi.SHAPE_QWEN3, abi.BF16, 3000, 2),
+    (abi.SHAPE_GRANITE, abi.F16, 2000, 34), (abi.SHAPE_GRANITE, abi.BF16, 1300, 9)])
+def test_a_query_of_another_dtype_is_rounded_to_the_caches(ctx, shape, dt, start, T, qdt):
+    """Sequence 1 of three, in a cache with room past the call."""
+    hq, hk, d, scale = HEADS[shape]
+    g = torch.Generator(device="cuda").manual_seed(start + T)
+    arena = rt.KvArena(ctx, shape, 1, 3, start + T + 77, dt)
+    k, v = (torch.randn((3, start + T + 50, hk, d), generator=g, device="cuda").to(TORCH[dt]) for _ in range(2))
+    q = (2 * torch.randn((T, hq, d), generator=g, device="cuda")).to(qdt)
+    out = torch.full((T, hq, d), float("nan"), device="cuda")
+    with rt.Graph(ctx) as graph:
+        rt.store_kv(graph, arena, 0, 0, k, v)
+        rt.prefill_attention(graph, arena, 0, start, q, out=out, sequence=1)
+    qf = q.float().to(TORCH[dt]).float().cpu().numpy()
+    kf, vf, out = k[1].float().cpu().numpy(), v[1].float().cpu().numpy(), out.cpu().numpy()
+    for t in sorted({0, 1, T // 2, T - 2, T - 1}):
+        n = start + t + 1
+        assert rel_err(out[t], attend64(qf[t], kf[:n], vf[:n], scale)) <= TOL_16, t
+    assert np.all(np.isfinite(out))

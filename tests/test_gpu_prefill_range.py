@@ -233,3 +233,20 @@ def test_a_workspace_of_a_long_prompt_serves_shorter_ones(ctx, kdt, vdt, capacit
         want = rt.prefill_attention(g, arena, 0, capacity - 127, q)
         out = rt.prefill_attention(g, arena, 0, capacity - 127, q, workspace=workspace)
     assert torch.equal(out, want)
+
+
+# ---- tiered values at the edges of tiles and chunks -------------------------------------------
+
+@pytest.mark.parametrize("window", [32, 128])
+@pytest.mark.parametrize("start,T", [(0, 64), (0, 65), (63, 66), (1, 255), (700, 128), (300, 640)])
+def test_tiered_values_at_edges(ctx, start, T, window):
+    k, v, q = inputs(start + T, T, start + T + window)
+    q *= 6
+    cap = start + T
+    arena = rt.KvArena(ctx, abi.SHAPE_GRANITE, 1, 1, cap, abi.F32, abi.I8_TIERED, value_window=window)
+    with rt.Graph(ctx) as g:
+        rt.store_kv(g, arena, 0, 0, k[None].cuda(), v[None].cuda())
+        out = rt.prefill_attention(g, arena, 0, start, q.cuda())
+        kk, vv = arena.gather(g, 0, 0, 0, cap)
+    check(out.cpu().numpy(), q, kk.float().cpu().numpy(), vv.float().cpu().numpy(), start,
+          sorted({0, 1, T // 2, max(0, T - 65), T - 1}))
