@@ -1008,10 +1008,11 @@ __global__ __launch_bounds__(64 * WAVES) void decode_mfma_kernel(DecodeArgs a) {
 // few-row prefill calls, a drafted block to verify.  A row attends all cached
 // positions but the last few, so a workgroup takes 16 / G rows at once,
 // their G heads each as the 16 columns of S^T (CB such column blocks over the
-// same tiles, rows_blocks), and streams its range of the K/V rows once for all of them (decode_mfma_kernel, one row a workgroup,
-// streams it once per row and leaves 16 - G columns idle).  Tiles, operands and
-// the two register sets are decode_mfma_body's; column (row t, head g) masks
-// positions past causal_start + t.  The partials are decode_combine_kernel's.
+// same tiles, rows_blocks), and streams its range of the K/V rows once for all
+// of them (decode_mfma_kernel, one row a workgroup, streams it once per row and
+// leaves 16 - G columns idle).  Tiles, operands and the two register sets are
+// decode_mfma_body's; column (row t, head g) masks positions past causal_start
+// + t.  The partials are decode_combine_kernel's.
 // Bound by the rate at which a CU pulls K/V from the caches behind it, and by
 // the merge: with one block, 15 tiles a wave take 26 us and 5 take 13, the same
 // with twice the waves a CU and with the workgroups that share a range on one

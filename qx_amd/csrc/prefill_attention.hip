@@ -27,21 +27,17 @@ __global__ __launch_bounds__(512, 1) void prefill_exact_pass_kernel(PrefillArgs 
 constexpr uint32_t kExactPassWgs = 256;
 
 // Causal rows on the split-K decode kernels, for short prompts on any cache
-// (and longer ones on Qwen-shape fp32 caches): every query row streams its own
-// prefix, split over the CUs like a decode.  That is quadratic in bytes for
-// long prompts but has no fixed cost beyond a decode's, while the pipelined
-// MFMA prefill (equal 16-bit K/V) first rewrites the layer's whole V prefix
-// into the f16 V^T scratch (bf16 and Qwen-shape caches; Granite f16 caches
-// skip that pass).  Measured per call (us; causal rows / pipelined, the
-// Granite figure with the pre-pass):
-// Qwen bf16 at 1020 cached positions 14 / 31 for 1-8 rows, 31 / 32 for 63;
-// at 8188, 42 / 56 for 16 rows; at 32764, 19 / 71 for one row, 71 / 71 for 8,
-// 142 / 69 for 16.  Granite f16 at 3840: 18 / 17 for 16 rows, 48 / 20 for 63.
+// (and longer ones on Qwen-shape fp32 caches): the cached prefix is streamed,
+// split over the CUs like a decode, once for every row or, on equal 16-bit
+// caches, once for the rows that share a workgroup (decode_mfma_rows_kernel).
+// That grows with rows x context but has no fixed cost beyond a decode's, while
+// the pipelined MFMA prefill (equal 16-bit K/V) first rewrites the layer's whole
+// V prefix into the f16 V^T scratch (bf16 and Qwen-shape caches; Granite f16
+// caches skip that pass).
 // Rows run on the decode kernels up to 8 of them, or, below 64, while rows x
 // context stays under the crossover measured against the kernel the call would
 // take otherwise (rows / tiled, us, 9-63 rows over 64-30000 cached positions,
-// each case timed both ways in one process; several rows share a workgroup,
-// decode_mfma_rows_kernel):
+// each case timed both ways):
 // - Qwen (960000 up to 32 rows, 500000 beyond): 30000 + 16 38.9 / 66.1, 16000
 //   + 32 41.2 / 50.1, 24000 + 32 54.4 / 59.6, 30000 + 24 54.0 / 66.2, 30000 +
 //   32 64.4 / 66.3, 8000 + 48 38.2 / 44.0, 12000 + 48 47.4 / 48.2, 8000 + 63
@@ -57,8 +53,6 @@ constexpr uint32_t kExactPassWgs = 256;
 // - the other Granite plans (tiered values with 16-bit keys): 40000;
 // - Qwen with tiered values (150000), whose decode rows keep splits toward
 //   2048 workgroups.
-// The former short-prompt kernel, one 8-head workgroup per kv head, took
-// 1.31 ms for 1-16 rows at 32764 Qwen positions.
 constexpr uint32_t kDecodeRowsAlways = 8;
 static bool rows_on_decode(const ShapeDims& s, int key_dtype, int value_dtype, uint32_t start, uint32_t tokens) {
     if (tokens <= kDecodeRowsAlways) return true;

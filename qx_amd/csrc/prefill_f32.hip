@@ -19,8 +19,10 @@
 //                         most 2^-24 of the product, what an fp32 product is
 //                         rounded by (2^-22 where x0 was cut off instead)
 //
-// Against 64 bits the result is as close as the fp32 matrix cores' was or
-// closer.
+// A tile's products are summed by themselves before they join the running sums,
+// so against 64 bits the result is closer than the fp32 matrix cores' was: 0.29
+// to 0.69 of its error over six K/V plans, prompts of 30 to 3063 positions and
+// scores spread by 0.1 to 4.
 //
 // Bound: a tile of Fp32KFp16V is 176 MFMAs a wave (2816 cycles of matrix core;
 // 8192 on the fp32 cores), beside the softmax and the split of the tile and of

@@ -1,5 +1,6 @@
-// Device helpers shared by the group-32 Q4 kernels (q4_projection.hip,
-// qwen_block.hip).  Layout and order: see q4_projection.hip.
+// Device helpers of the group-32 Q4 kernels: the Granite rows' fold and tree
+// (q4_projection.hip, which has layout and order), and the conversions that
+// qwen_block.hip shares with it.
 #pragma once
 #include "common.h"
 
@@ -43,9 +44,6 @@ __device__ __forceinline__ float q4_fold(const uint8_t* codes, float scale, cons
     return acc;
 }
 
-// The 32-group case (a full 1024-column chunk): the batched fold.
-__device__ __forceinline__ float q4_fold32(const uint8_t* codes, float scale, const float* in, int l, float acc);
-
 // The scale of group g (g < 32 within a 32-group block) for this lane's row:
 // lanes 0-31 hold row A's scales (lane g: group g), lanes 32-63 row B's, so
 // two readlanes and a select give every lane its row's value without LDS.
@@ -55,59 +53,38 @@ __device__ __forceinline__ float half_scale(float sc, int g, bool upper) {
     return upper ? b : a;
 }
 
-// The lane's fold over NG groups (NG a multiple of 32) of its half-wave's
-// row, starting from `acc`: `codes` holds the row's NG staged groups (group
-// g at byte 16 g), sc[j] the lane's scale of group 32 j + l, `in` the staged
-// input.  Group by group, fma into one accumulator (the reference lane's
-// order); code bytes and inputs are read from LDS a batch of 16 groups ahead
-// of their use so the chain does not wait on LDS.  Fully unrolled: a rolled
-// batch loop measured slower.  The whole wave must run it (readlane).
-template <int NG>
-__device__ __forceinline__ float q4_fold_n(const uint8_t* codes, const float (&sc)[NG / 32], const float* in, int l,
-                                           float acc) {
+// The lane's fold over the 32 groups of a full 1024-column chunk of its
+// half-wave's row, starting from `acc`: `codes` holds the staged groups (group
+// g at byte 16 g), `scale` the lane's scale of group l, `in` the staged input.
+// Group by group, fma into one accumulator (the reference lane's order); code
+// bytes and inputs are read from LDS a batch of 16 groups ahead of their use so
+// the chain does not wait on LDS.  Fully unrolled: a rolled batch loop measured
+// slower.  The whole wave must run it (readlane).
+__device__ __forceinline__ float q4_fold32(const uint8_t* codes, float scale, const float* in, int l, float acc) {
     constexpr int B = 16;
-    static_assert(NG % 32 == 0, "whole 32-group blocks");
     const int shift = (l & 1) * 4;
     const bool upper = (__lane_id() & 32) != 0;
-    uint32_t cb[B];
-    float xin[B];
-#pragma unroll
-    for (int i = 0; i < B; ++i) {
-        cb[i] = codes[i * 16 + (l >> 1)];
-        xin[i] = in[i * 32 + l];
-    }
-#pragma unroll
-    for (int b = 0; b < NG / B; ++b) {
-        uint32_t ncb[B];
-        float nx[B];
-        if (b + 1 < NG / B) {
-#pragma unroll
-            for (int i = 0; i < B; ++i) {
-                ncb[i] = codes[((b + 1) * B + i) * 16 + (l >> 1)];
-                nx[i] = in[((b + 1) * B + i) * 32 + l];
-            }
-        }
+    uint32_t cb[2][B];
+    float xin[2][B];
+    auto read = [&](int b) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < B; ++i) {
-            const int g = b * B + i;
-            const uint32_t code = (cb[i] >> shift) & 0xfu;
-            const float w = (float)((int)code - 7) * half_scale(sc[g / 32], g % 32, upper);
-            acc = __builtin_fmaf(w, xin[i], acc);
+            cb[b][i] = codes[(b * B + i) * 16 + (l >> 1)];
+            xin[b][i] = in[(b * B + i) * 32 + l];
         }
-        if (b + 1 < NG / B) {
+    };
+    read(0);
 #pragma unroll
-            for (int i = 0; i < B; ++i) {
-                cb[i] = ncb[i];
-                xin[i] = nx[i];
-            }
+    for (int b = 0; b < 2; ++b) {
+        if (b == 0) read(1);
+#pragma unroll
+        for (int i = 0; i < B; ++i) {
+            const uint32_t code = (cb[b][i] >> shift) & 0xfu;
+            const float w = (float)((int)code - 7) * half_scale(scale, b * B + i, upper);
+            acc = __builtin_fmaf(w, xin[b][i], acc);
         }
     }
     return acc;
-}
-
-__device__ __forceinline__ float q4_fold32(const uint8_t* codes, float scale, const float* in, int l, float acc) {
-    const float sc[1] = {scale};
-    return q4_fold_n<32>(codes, sc, in, l, acc);
 }
 
 __device__ __forceinline__ float round_f16(float x) { return (float)(_Float16)x; }
