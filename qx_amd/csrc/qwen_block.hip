@@ -59,7 +59,7 @@ __device__ __forceinline__ float qwen_inverse_rms(float total) {
 // (0x6400 | n is 1024 + n), so the inputs are paired the same way.
 //
 // 10.6 MB of codes a layer: both kernels are bound by their dispatch and one
-// round trip to HBM (4.8 and 4.0 us traced; the codes alone take 0.9 and 0.7).
+// round trip to HBM (4.5 and 4.0 to 4.5 us traced; the codes alone take 0.9 and 0.7).
 // Measured, 48 layers at 32768 positions, us a token: a row's codes dealt
 // back to the reference's 32 lanes through LDS (two LDS reads and eight VALU
 // instructions a value) 1565; a group per lane, each wave normalising the
